@@ -817,6 +817,13 @@ void check_tree_kernels() {
     check_kernel_resources((const void*)gj_update_kernel, "gj_update_kernel");
     check_kernel_resources((const void*)gj_perm_kernel, "gj_perm_kernel");
     check_kernel_resources((const void*)gj_gather_kernel, "gj_gather_kernel");
+    check_kernel_resources((const void*)inv_wave_kernel<1>, "inv_wave_kernel<1>");
+    check_kernel_resources((const void*)inv_wave_kernel<2>, "inv_wave_kernel<2>");
+    check_kernel_resources((const void*)inv_wave_kernel<4>, "inv_wave_kernel<4>");
+    check_kernel_resources((const void*)inv_small_kernel<8>, "inv_small_kernel<8>");
+    check_kernel_resources((const void*)inv_pivot_kernel, "inv_pivot_kernel");
+    check_kernel_resources((const void*)inv_mult_kernel, "inv_mult_kernel");
+    check_kernel_resources((const void*)inv_update_kernel, "inv_update_kernel");
     check_kernel_resources((const void*)tree_assemble_kernel, "tree_assemble_kernel");
     check_kernel_resources((const void*)tree_coarsen_kernel, "tree_coarsen_kernel");
     check_kernel_resources((const void*)tree_up_gather_kernel, "tree_up_gather_kernel");
@@ -841,12 +848,11 @@ void do_build(ef_mesh_s* M, const ef_coeffs& c) {
     M->Sar.ensure(std::max<long long>(P.S_elems, 1));
     M->Xiar.ensure(std::max<long long>(P.Xi_elems, 1));
     M->wX.ensure(std::max<long long>(P.work_X, 1));
-    M->gjd.ensure(std::max<long long>(P.gj_d, 1));
-    M->gji.ensure(std::max<long long>(P.gj_i, 1));
-    M->info.ensure(std::max(P.ninternal, 1));
+    const size_t ngroups = P.groups.size(), ninfo = (size_t)P.ninternal + ngroups;
+    M->info.ensure(std::max<size_t>(ninfo, 1));
     // the merge descriptors depend only on these addresses and on the leaf DtN each leaf
     // reads: planned again only when one of them moved
-    std::vector<const void*> sig = {M->Tar.p, M->Sar.p, M->Xiar.p, M->wX.p, M->gjd.p, M->gji.p, M->info.p,
+    std::vector<const void*> sig = {M->Tar.p, M->Sar.p, M->Xiar.p, M->wX.p, M->info.p,
                                     (const void*)(intptr_t)(M->precision + 1)};
     for (size_t li = 0; li < P.leaves.size(); li++) sig.push_back(leaf_T_ptr(M, (int)li));
     if (sig != M->plan_sig) {
@@ -879,25 +885,42 @@ void do_build(ef_mesh_s* M, const ef_coeffs& c) {
     }
     if (sync_check()) EF_HIP(hipStreamSynchronize(s));
     if (M->bstore.pending()) throw EfError(EF_ERR_INTERNAL, "merge descriptors staged but not uploaded");
-    // merges, deepest level first (post-order dependencies)
-    EF_HIP(hipMemsetAsync(M->info.p, 0, sizeof(int) * std::max(P.ninternal, 1), s));
-    for (size_t gi = 0; gi < P.groups.size(); gi++) {
-        const Group& g = P.groups[gi];
-        const GroupPlan& gp = M->gplans[gi];
-        const int n = g.n, B = (int)g.nodes.size(), m = 4 * n;
-        for (size_t t = 0; t < gp.csteps.size(); t++) {
-            const long long out = 4LL * gp.csteps_maxm[t] * gp.csteps_maxm[t];
-            EF_LAUNCH("tree_coarsen_kernel", tree_coarsen_kernel, dim3(blocks_for(out), gp.csteps_cnt[t]), dim3(256), s,
-                      gp.csteps[t]);
+    // merges, deepest level first (post-order dependencies), from group gi0: X inverted in natural
+    // order, or with row exchanges when `pivoted`
+    auto merges = [&](size_t gi0, bool pivoted) {
+        for (size_t gi = gi0; gi < ngroups; gi++) {
+            const Group& g = P.groups[gi];
+            const GroupPlan& gp = M->gplans[gi];
+            const int n = g.n, B = (int)g.nodes.size(), m = 4 * n;
+            for (size_t t = 0; t < gp.csteps.size(); t++) {
+                const long long out = 4LL * gp.csteps_maxm[t] * gp.csteps_maxm[t];
+                EF_LAUNCH("tree_coarsen_kernel", tree_coarsen_kernel, dim3(blocks_for(out), gp.csteps_cnt[t]), dim3(256), s,
+                          gp.csteps[t]);
+            }
+            EF_LAUNCH("tree_assemble_kernel", tree_assemble_kernel, dim3(blocks_for(80LL * n * n), B), dim3(256), s, gp.asmd);
+            if (pivoted)
+                run_gj_inverse(M->wX.p, M->Xiar.p + g.Xi0, m, B, gj_work(M, m, B), M->info.p + g.info0, s);
+            else  // the group's S (2 m^2 each, formed next) is the work
+                run_inverse(M->wX.p, M->Xiar.p + g.Xi0, m, B, M->Sar.p + P.nodes[g.nodes[0]].S_off,
+                            M->info.p + P.ninternal + gi, s);
+            run_gemm(gp.gS, s);
+            run_gemm(gp.gT, s);
         }
-        EF_LAUNCH("tree_assemble_kernel", tree_assemble_kernel, dim3(blocks_for(80LL * n * n), B), dim3(256), s, gp.asmd);
-        run_gj_inverse(M->wX.p, M->Xiar.p + g.Xi0, m, B, gj_work(M, m, B), M->info.p + g.info0, s);
-        run_gemm(gp.gS, s);
-        run_gemm(gp.gT, s);
-    }
-    // zero pivots of any merge: one read at the end of the stage
-    std::vector<int> info(std::max(P.ninternal, 1), 0);
+    };
+    EF_HIP(hipMemsetAsync(M->info.p, 0, sizeof(int) * std::max<size_t>(ninfo, 1), s));
+    merges(0, false);
+    // flags of the groups' inversions and zero pivots of any merge: one read at the end of the stage
+    std::vector<int> info(std::max<size_t>(ninfo, 1), 0);
     efk::copy_d2h(info.data(), M->info.p, sizeof(int) * info.size(), s);
+    for (size_t gi = 0; gi < ngroups; gi++)
+        if (info[P.ninternal + gi] != 0) {
+            // a multiplier too large for the natural order: this group and all above it again, pivoted
+            M->gjd.ensure(std::max<long long>(P.gj_d, 1));
+            M->gji.ensure(std::max<long long>(P.gj_i, 1));
+            merges(gi, true);
+            efk::copy_d2h(info.data(), M->info.p, sizeof(int) * info.size(), s);
+            break;
+        }
     for (size_t gi = 0; gi < P.groups.size(); gi++) {
         const Group& g = P.groups[gi];
         for (size_t b = 0; b < g.nodes.size(); b++)
@@ -1385,26 +1408,38 @@ void do_solve_once(ef_mesh_s* M, const double* f_dev, const double* r_dev, const
         M->rootA.ensure((size_t)m * m);
         M->rootAi.ensure((size_t)m * m);
         M->rootrhs.ensure((size_t)m * k);
-        M->rootgj.ensure(gj_work_doubles(m, 1));
+        M->rootgj.ensure(std::max(gj_work_doubles(m, 1), inv_work_doubles(m, 1)));
         M->rootgji.ensure(gj_work_ints(m, 1));
-        M->rootinfo.ensure(1);
+        M->rootinfo.ensure(2);
         const double* Troot = full_T_ptr(M, 0);
         const double* hroot = (root.leaf || M->homogeneous_rhs) ? nullptr : V + root.h_off;
-        EF_LAUNCH("tree_root_robin_kernel", tree_root_robin_kernel, dim3(blocks_for((long long)m * m + (long long)m * k)),
-                  dim3(256), s, Troot, a_dev, b_dev, r_dev, hroot, M->rootA.p, M->rootrhs.p, m, k, P.vec_rows);
-        GJWork w;
-        double* d = M->rootgj.p;
-        w.wb = d; d += (size_t)m * m;
-        w.Pinv = d; d += (size_t)GJ_NB * GJ_NB;
-        w.Mm = d;
-        int* ii = M->rootgji.p;
-        w.cand = ii; ii += (size_t)GJ_MAXCH * GJ_NB;
-        w.cfin = ii; ii += (size_t)GJ_NB;
-        w.src = ii; ii += (size_t)m;
-        w.ipiv = ii; ii += (size_t)m;
-        w.prow = ii;
-        EF_HIP(hipMemsetAsync(M->rootinfo.p, 0, sizeof(int), s));
-        run_gj_inverse(M->rootA.p, M->rootAi.p, m, 1, w, M->rootinfo.p, s);
+        int info[2] = {0, 0};  // zero pivot, multiplier too large for the natural order
+        EF_HIP(hipMemsetAsync(M->rootinfo.p, 0, 2 * sizeof(int), s));
+        auto system = [&] {
+            EF_LAUNCH("tree_root_robin_kernel", tree_root_robin_kernel,
+                      dim3(blocks_for((long long)m * m + (long long)m * k)), dim3(256), s, Troot, a_dev, b_dev, r_dev, hroot,
+                      M->rootA.p, M->rootrhs.p, m, k, P.vec_rows);
+        };
+        system();
+        run_inverse(M->rootA.p, M->rootAi.p, m, 1, M->rootgj.p, M->rootinfo.p + 1, s);
+        efk::copy_d2h(info, M->rootinfo.p, 2 * sizeof(int), s);
+        if (info[1]) {
+            GJWork w;
+            double* d = M->rootgj.p;
+            w.wb = d; d += (size_t)m * m;
+            w.Pinv = d; d += (size_t)GJ_NB * GJ_NB;
+            w.Mm = d;
+            int* ii = M->rootgji.p;
+            w.cand = ii; ii += (size_t)GJ_MAXCH * GJ_NB;
+            w.cfin = ii; ii += (size_t)GJ_NB;
+            w.src = ii; ii += (size_t)m;
+            w.ipiv = ii; ii += (size_t)m;
+            w.prow = ii;
+            system();
+            run_gj_inverse(M->rootA.p, M->rootAi.p, m, 1, w, M->rootinfo.p, s);
+            efk::copy_d2h(info, M->rootinfo.p, sizeof(int), s);
+            if (info[0]) throw EfError(EF_ERR_SINGULAR, "zero pivot in the root boundary system");
+        }
         TreeGemm p{};
         p.A0 = M->rootAi.p; p.lda0 = m; p.K0 = m; p.alpha0 = 1.0;
         p.B0 = M->rootrhs.p; p.ldb0 = 1; p.bcs = m;
@@ -1414,9 +1449,7 @@ void do_solve_once(ef_mesh_s* M, const double* f_dev, const double* r_dev, const
         GemmLaunch g = plan_gemm(std::vector<TreeGemm>{p}, k <= 16 ? 1 : 2, tmp, s);
         tmp.flush(s);
         run_gemm(g, s);
-        int info = 0;
-        efk::copy_d2h(&info, M->rootinfo.p, sizeof(int), s);
-        if (info) throw EfError(EF_ERR_SINGULAR, "zero pivot in the root boundary system");
+        EF_HIP(hipStreamSynchronize(s));  // the launch's descriptors are freed here
     }
     downward();
 }

@@ -870,6 +870,540 @@ __global__ void __launch_bounds__(256) gj_gather_kernel(GJArgs a) {
 }
 
 // ---------------------------------------------------------------------------------------
+// Inversion without row exchanges
+// ---------------------------------------------------------------------------------------
+// The interface systems of elliptic problems are definite up to row signs (sums of the children's
+// boundary operators), so Gauss-Jordan needs no pivot search on them: over adaptive, variable and
+// uniform meshes with lambda <= 0 the largest multiplier is 1.3, and the inverse's residual equals
+// a pivoted LU's.  These kernels eliminate in natural order and check every multiplier against
+// INV_LMAX; one beyond it (an indefinite system, a zero pivot, a NaN) sets *flag, and the caller
+// inverts again with the pivoted kernels above.  What bounds the pivoted path is its 32-column panel,
+// a chain of 32 dependent column searches (52 us per launch): the inversions of the adaptive
+// Poisson mesh (1,937 merges, m = 64 .. 1024) took 7.4 ms of GPU time with it and take 1.2 ms so,
+// those of 1,024 leaves of 32 x 32 cells 12.9 and 2.3 ms.
+
+// x, opaque to the compiler: what is computed from it is computed after this point
+__device__ inline int formed_here(int x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+s"(x));
+#endif
+    return x;
+}
+
+// 1 / x: hardware estimate and two Newton steps (relative error about 1 ulp; inf or NaN at 0)
+__device__ inline double inv_rcp(double x) {
+    double rc = __builtin_amdgcn_rcp(x);
+    rc = fma(rc, fma(-x, rc, 1.0), rc);
+    return fma(rc, fma(-x, rc, 1.0), rc);
+}
+
+// Gauss-Jordan on a 16 x 16 block by one wave, in place, in the accumulator layout (slot v of lane
+// (q, r) is element (4v + q, r)), four columns at a time: the rows 4g .. 4g + 3 of group g are
+// slot g.  Through LDS (buf: 16 x 18) every lane gets the 4 x 4 pivot block P, its own column of
+// those rows (a unit vector in the pivot columns) and one entry of the pivot columns, solves
+// P x = column in registers -- x_q is its entry of the new rows -- and one MFMA subtracts the pivot
+// columns times the new rows from all others.  Column by column, with the pivot row and column
+// broadcast across lanes, a block took 6,300 cycles (393 a column, a chain of reciprocal,
+// broadcasts and selects); so it takes a third of that.
+// Checked: the multipliers inside P and those of the other rows.
+// bg(g) issues products of the caller's that run on the matrix cores meanwhile.
+template <class BG>
+__device__ inline void inv16(td4& D, double* buf, bool& ok, BG&& bg) {
+    const int lane = threadIdx.x & 63, q = lane >> 4, r = lane & 15;
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int v = 0; v < 4; v++) buf[(4 * v + q) * 18 + r] = D[v];
+        __builtin_amdgcn_wave_barrier();
+        double P[4][4], x[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const td2 u = *(const td2*)(buf + (4 * g + i) * 18 + 4 * g), w = *(const td2*)(buf + (4 * g + i) * 18 + 4 * g + 2);
+            P[i][0] = u[0]; P[i][1] = u[1]; P[i][2] = w[0]; P[i][3] = w[1];
+            x[i] = buf[(4 * g + i) * 18 + r];
+        }
+        const double a = -buf[r * 18 + 4 * g + q];
+        __builtin_amdgcn_wave_barrier();
+        bg(g);
+        const bool pcol = (r >> 2) == g;  // a pivot column
+#pragma unroll
+        for (int i = 0; i < 4; i++) x[i] = pcol ? ((r & 3) == i ? 1.0 : 0.0) : x[i];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {  // LU of P, its inverse diagonal in P(j, j); x forward
+            P[j][j] = inv_rcp(P[j][j]);
+#pragma unroll
+            for (int i = j + 1; i < 4; i++) {
+                const double l = P[i][j] * P[j][j];
+                ok = ok & (fabs(l) <= INV_LMAX);
+#pragma unroll
+                for (int c = j + 1; c < 4; c++) P[i][c] = fma(-l, P[j][c], P[i][c]);
+                x[i] = fma(-l, x[j], x[i]);
+            }
+        }
+#pragma unroll
+        for (int j = 3; j >= 0; j--) {  // and back
+#pragma unroll
+            for (int c = j + 1; c < 4; c++) x[j] = fma(-P[j][c], x[c], x[j]);
+            x[j] *= P[j][j];
+        }
+        const double xq = q < 2 ? (q == 0 ? x[0] : x[1]) : (q == 2 ? x[2] : x[3]);
+        td4 C;
+#pragma unroll
+        for (int v = 0; v < 4; v++) C[v] = pcol ? 0.0 : D[v];
+        C = mfma_f64(a, xq, C);
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            if (v != g) ok = ok & (!pcol | (fabs(C[v]) <= INV_LMAX));
+            D[v] = v == g ? xq : C[v];
+        }
+    }
+}
+
+// LDS of an inversion by WAVES waves: the pivot tile row of a step (its diagonal tile already
+// inverted) by step parity, and one 16 x 16 transposition tile per wave
+template <int MT, int WAVES>
+struct InvShared {
+    double rp[2][MT][4][64];
+    alignas(16) double tr[WAVES][16 * 18];
+};
+
+// In-place inversion of mt x mt tiles of 16 x 16 (mt <= MT <= WAVES): wave w holds tile row w, tile
+// j in T[j], in the accumulator layout.  Before step kb wave kb has inverted its diagonal tile and
+// published its tile row; after the step's one barrier every other wave forms L = A_wk P^-1 and
+// its transpose from one transposed copy of its own tile and subtracts L times the published row,
+// and wave kb multiplies its row by P^-1.  Wave kb + 1 updates its diagonal tile first and inverts
+// it while the rest of its row is updated, which leaves one tile update and one inversion between
+// two barriers.  (OVERLAP: the inversion and the row's other products are interleaved, for a lone
+// workgroup; without it they follow one another in fewer registers, so that more workgroups
+// share a CU.)  An accumulator tile is the B operand of the next product as it stands, and the
+// accumulator of L^T is the A operand of L.
+template <bool OVERLAP, int MT, int WAVES>
+__device__ inline void inv_tiles(td4 (&T)[MT], int mt, InvShared<MT, WAVES>& sh, bool& ok) {
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    const int q = lane >> 4, r = lane & 15;
+    double* tr = sh.tr[wave];
+    auto tile = [&](int k) {  // T[k], k uniform
+        td4 D = T[0];
+#pragma unroll
+        for (int j = 1; j < MT; j++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) D[v] = (j == k) ? T[j][v] : D[v];
+        return D;
+    };
+    auto put = [&](int k, const td4& D) {
+#pragma unroll
+        for (int j = 0; j < MT; j++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) T[j][v] = (j == k) ? D[v] : T[j][v];
+    };
+    auto publish = [&](int k) {
+#pragma unroll
+        for (int j = 0; j < MT; j++)
+            if (j < mt)
+#pragma unroll
+                for (int v = 0; v < 4; v++) sh.rp[k & 1][j][v][lane] = T[j][v];
+    };
+    if (wave == 0) {
+        inv16(T[0], tr, ok, [](int) {});
+        publish(0);
+    }
+#pragma unroll(OVERLAP ? MT : 1)
+    for (int kb = 0; kb < MT; kb++) {
+        if (kb >= mt) break;
+        const td4 D = tile(kb);
+        // the own tile's transpose: a[s] = D(r, 4s + q), an A operand
+#pragma unroll
+        for (int v = 0; v < 4; v++) tr[(4 * v + q) * 18 + r] = D[v];
+        __builtin_amdgcn_wave_barrier();
+        double a[4];
+#pragma unroll
+        for (int s = 0; s < 4; s++) a[s] = tr[r * 18 + 4 * s + q];
+        __syncthreads();
+        const double (&rp)[MT][4][64] = sh.rp[kb & 1];
+        if (wave == kb) {
+#pragma unroll
+            for (int j = 0; j < MT; j++) {
+                if (j >= mt || j == kb) continue;
+                td4 x = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+                for (int s = 0; s < 4; s++) x = mfma_f64(a[s], T[j][s], x);
+                T[j] = x;
+            }
+        } else if (wave < mt) {
+            td4 Lt = {0.0, 0.0, 0.0, 0.0}, L = Lt;
+            double p[4];
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                p[s] = rp[kb][s][lane];
+                Lt = mfma_f64(p[s], a[s], Lt);
+            }
+#pragma unroll
+            for (int v = 0; v < 4; v++) ok = ok & (fabs(Lt[v]) <= INV_LMAX);
+            // tile j minus L times the published tile; column kb: -A P^-1
+            auto update = [&](td4& X, int j) {
+#pragma unroll
+                for (int s = 0; s < 4; s++) X = mfma_f64(-Lt[s], rp[j][s][lane], X);
+                if (!OVERLAP) __builtin_amdgcn_sched_barrier(0);  // one tile's operands in registers at a time
+            };
+            auto column = [&] {
+#pragma unroll
+                for (int s = 0; s < 4; s++) L = mfma_f64(-a[s], p[s], L);
+            };
+            if (wave == kb + 1) {
+                td4 X = tile(kb + 1);
+                update(X, kb + 1);
+                auto rest = [&](int g) {
+#pragma unroll
+                    for (int j = 0; j < MT; j++)
+                        if ((j & 3) == g && j < mt && j != kb && j != kb + 1) update(T[j], j);
+                };
+                column();
+                put(kb, L);
+                if constexpr (OVERLAP) {
+                    inv16(X, tr, ok, rest);
+                } else {
+                    inv16(X, tr, ok, [](int) {});
+#pragma unroll
+                    for (int g = 0; g < 4; g++) rest(g);
+                }
+                put(kb + 1, X);
+                publish(kb + 1);
+            } else {
+#pragma unroll
+                for (int j = 0; j < MT; j++)
+                    if (j < mt && j != kb) update(T[j], j);
+                column();
+                put(kb, L);
+            }
+        }
+    }
+}
+
+// Whole inverses of matrices of order m <= 16 MT <= 64, one wave each (four independent waves per
+// workgroup, no barrier): tile (i, j) in T[i][j], the steps of inv_tiles with every tile at hand.
+// A launch has hundreds of such matrices; with a workgroup of four waves each, one or two per CU
+// for the registers, the adaptive Poisson mesh's matrices of order 64 took 140 us, so 85 us.
+template <int MT>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8)))
+inv_wave_kernel(const double* __restrict__ A, double* __restrict__ Ai, int m, int B, int* flag) {
+    __shared__ __attribute__((aligned(16))) double tr_all[4][16 * 18];
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    const int q = lane >> 4, r = lane & 15, b = (int)blockIdx.x * 4 + wave;
+    if (b >= B) return;  // uniform per wave; no barrier below
+    double* tr = tr_all[wave];
+    const auto* Ab = gmem(A) + (long long)b * m * m;
+    td4 T[MT][MT];
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const int row = 16 * i + 4 * v + q;
+            const auto* p = Ab + (long long)min(row, m - 1) * m;
+#pragma unroll
+            for (int j = 0; j < MT; j++) {
+                const int col = 16 * j + r;
+                const double x = p[min(col, m - 1)];
+                T[i][j][v] = (row < m && col < m) ? x : (row == col ? 1.0 : 0.0);
+            }
+        }
+    bool ok = true;
+    auto transpose = [&](const td4& D, double (&a)[4]) {  // a[s] = D(r, 4s + q), an A operand
+#pragma unroll
+        for (int v = 0; v < 4; v++) tr[(4 * v + q) * 18 + r] = D[v];
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int s = 0; s < 4; s++) a[s] = tr[r * 18 + 4 * s + q];
+        __builtin_amdgcn_wave_barrier();
+    };
+#pragma unroll
+    for (int kb = 0; kb < MT; kb++) {
+        if (16 * kb >= m) continue;  // (identity beyond)
+        inv16(T[kb][kb], tr, ok, [](int) {});
+        const td4 P = T[kb][kb];
+        double a[4];
+#pragma unroll
+        for (int i = 0; i < MT; i++) {
+            if (i == kb) continue;
+            transpose(T[i][kb], a);
+            td4 Lt = {0.0, 0.0, 0.0, 0.0}, L = Lt;
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                Lt = mfma_f64(P[s], a[s], Lt);
+                L = mfma_f64(-a[s], P[s], L);
+            }
+            T[i][kb] = L;
+#pragma unroll
+            for (int v = 0; v < 4; v++) ok = ok & (fabs(Lt[v]) <= INV_LMAX);
+#pragma unroll
+            for (int j = 0; j < MT; j++)
+                if (j != kb)
+#pragma unroll
+                    for (int s = 0; s < 4; s++) T[i][j] = mfma_f64(-Lt[s], T[kb][j][s], T[i][j]);
+        }
+        transpose(P, a);
+#pragma unroll
+        for (int j = 0; j < MT; j++) {
+            if (j == kb) continue;
+            td4 x = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int s = 0; s < 4; s++) x = mfma_f64(a[s], T[kb][j][s], x);
+            T[kb][j] = x;
+        }
+    }
+    const int ms = formed_here(m);  // the stores' addresses are not kept from the loads
+    auto* Ib = gmem(Ai) + (long long)b * ms * ms + r;
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const int row = 16 * i + 4 * v + q;
+#pragma unroll
+            for (int j = 0; j < MT; j++)
+                if (row < ms && 16 * j + r < ms) Ib[(long long)row * ms + 16 * j] = T[i][j][v];
+        }
+    if (!ok) *flag = 1;
+}
+
+template __global__ void inv_wave_kernel<1>(const double*, double*, int, int, int*);
+template __global__ void inv_wave_kernel<2>(const double*, double*, int, int, int*);
+template __global__ void inv_wave_kernel<4>(const double*, double*, int, int, int*);
+
+// Whole inverses of matrices of order m <= 16 MT, one workgroup of MT waves each (64 < m <= 128).
+template <int MT>
+__global__ void __launch_bounds__(64 * MT) __attribute__((amdgpu_waves_per_eu(2, 8)))
+inv_small_kernel(const double* __restrict__ A, double* __restrict__ Ai, int m,
+                                                            int* flag) {
+    __shared__ InvShared<MT, MT> sh;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    const int q = lane >> 4, r = lane & 15, mt = (m + 15) / 16;
+    const auto* Ab = gmem(A) + (long long)blockIdx.x * m * m;
+    auto* Ib = gmem(Ai) + (long long)blockIdx.x * m * m;
+    td4 T[MT];
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        const int row = 16 * wave + 4 * v + q;
+        const auto* p = Ab + (long long)min(row, m - 1) * m;
+#pragma unroll
+        for (int j = 0; j < MT; j++) {
+            const int col = 16 * j + r;
+            const double x = p[min(col, m - 1)];
+            T[j][v] = (row < m && col < m) ? x : (row == col ? 1.0 : 0.0);
+        }
+    }
+    bool ok = true;
+    inv_tiles<false>(T, mt, sh, ok);
+    const int ms = formed_here(m);  // the stores' addresses are not kept from the loads
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        const int row = 16 * wave + 4 * v + q;
+        auto* p = Ib + (long long)row * ms + r;
+#pragma unroll
+        for (int j = 0; j < MT; j++)
+            if (row < ms && 16 * j + r < ms) p[16 * j] = T[j][v];
+    }
+    if (!ok) *flag = 1;
+}
+
+template __global__ void inv_small_kernel<8>(const double*, double*, int, int*);
+
+// Larger orders, INV_NB = 64 columns per step, two launches a step: the multipliers M (m x INV_NB,
+// inv_mult_kernel) and the rank-64 update (inv_update_kernel), whose first workgroup goes on to
+// invert the next step's pivot block while the others update the rest of the matrix.  A step is
+// bound by that chain (update one block, 64 dependent columns, multipliers): 17 + 6 us a step at
+// m <= 1024.  Inverting the pivot block in every workgroup of the multipliers instead, with the
+// inversion in the open, took 24 + 8 us.
+
+// P^-1 of the pivot block (nb x nb, here in strips of tiles), zero beyond nb, into Pn (INV_NB x INV_NB)
+__device__ inline void inv_pivot_block(td4 (&T)[INV_NB / 16], int nb, InvShared<INV_NB / 16, 4>& sh, double* Pn, int* flag) {
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    const int q = lane >> 4, r = lane & 15;
+    bool ok = true;
+    inv_tiles<true>(T, (nb + 15) / 16, sh, ok);
+#pragma unroll
+    for (int j = 0; j < INV_NB / 16; j++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const int row = 16 * wave + 4 * v + q, col = 16 * j + r;
+            gmem(Pn)[row * INV_NB + col] = (row < nb && col < nb) ? T[j][v] : 0.0;
+        }
+    if (!ok) *flag = 1;
+}
+
+// the first step's pivot block, one workgroup per matrix
+__global__ void __launch_bounds__(256) inv_pivot_kernel(const double* __restrict__ A, double* __restrict__ Pn, int m,
+                                                        int* flag) {
+    __shared__ InvShared<INV_NB / 16, 4> sh;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    const int q = lane >> 4, r = lane & 15;
+    const auto* Ab = gmem(A) + (long long)blockIdx.x * m * m;
+    td4 T[INV_NB / 16];
+#pragma unroll
+    for (int j = 0; j < INV_NB / 16; j++)
+#pragma unroll
+        for (int v = 0; v < 4; v++)  // m > INV_NB
+            T[j][v] = Ab[(long long)(16 * wave + 4 * v + q) * m + 16 * j + r];
+    inv_pivot_block(T, INV_NB, sh, Pn + (long long)blockIdx.x * INV_NB * INV_NB, flag);
+}
+
+// M = P^-1 on the pivot rows, -A P^-1 elsewhere (zero beyond the matrix's columns): one wave per
+// 16 rows x 32 columns, all operands loaded before the products.
+__global__ void __launch_bounds__(512) inv_mult_kernel(const double* __restrict__ A, double* __restrict__ Mm,
+                                                       const double* __restrict__ Pn, int m, int k, int* flag) {
+    constexpr int MT = INV_NB / 16;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    const int q = lane >> 4, r = lane & 15;
+    const int nb = min(INV_NB, m - k), row0 = (int)blockIdx.x * 64 + 16 * (wave & 3), j0 = 2 * (wave >> 2);
+    const auto* Ab = gmem(A) + (long long)blockIdx.y * m * m;
+    const auto* Pb = gmem(Pn) + (long long)blockIdx.y * INV_NB * INV_NB;
+    auto* Mb = gmem(Mm) + (long long)blockIdx.y * m * INV_NB;
+    const bool pivot_rows = (int)blockIdx.x * 64 == k;  // uniform: k is a multiple of 64
+    td4 x[2];
+    if (pivot_rows) {
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) x[j][v] = Pb[(row0 - k + 4 * v + q) * INV_NB + 16 * (j0 + j) + r];
+    } else {
+        // lane group q takes columns 16 t + 4q + s at step s; m, nb are multiples of 4
+        td2 a[MT][2];
+        double b[MT][2][4];
+        const auto* ar = Ab + (long long)min(row0 + r, m - 1) * m + k;
+#pragma unroll
+        for (int t = 0; t < MT; t++) {
+            const int c = min(16 * t + 4 * q, nb - 4);  // past nb: times the zero rows of P^-1
+            a[t][0] = *(const EF_GLOBAL td2*)(ar + c);
+            a[t][1] = *(const EF_GLOBAL td2*)(ar + c + 2);
+        }
+#pragma unroll
+        for (int t = 0; t < MT; t++)
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int s = 0; s < 4; s++) b[t][j][s] = Pb[(16 * t + 4 * q + s) * INV_NB + 16 * (j0 + j) + r];
+        x[0] = x[1] = td4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int t = 0; t < MT; t++)
+#pragma unroll
+            for (int s = 0; s < 4; s++)
+#pragma unroll
+                for (int j = 0; j < 2; j++) x[j] = mfma_f64(-a[t][s >> 1][s & 1], b[t][j][s], x[j]);
+        bool ok = true;
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) ok = ok & (fabs(x[j][v]) <= INV_LMAX);
+        if (!ok) *flag = 1;
+    }
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const int row = row0 + 4 * v + q;
+            if (row < m) Mb[(long long)row * INV_NB + 16 * (j0 + j) + r] = x[j][v];
+        }
+}
+
+// The step's update into the other buffer: Wb = Wa + M Wa(pivot rows), Wb = M Wa(pivot rows) on the
+// pivot rows themselves, and the pivot columns are M.  One workgroup per 64 x 64 block, a wave per
+// 32 x 32 quarter; all of a quarter's operands are loaded before its products (K is 64), so a wave
+// waits for memory once.  Workgroup 0 of a matrix takes the next pivot block and inverts it (Pn).
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8)))
+inv_update_kernel(const double* __restrict__ Wa, double* __restrict__ Wb,
+                                                         const double* __restrict__ Mm, double* __restrict__ Pn, int m,
+                                                         int k, int* flag) {
+    constexpr int MT = INV_NB / 16;
+    __shared__ union {
+        InvShared<MT, 4> inv;
+        double blk[MT][MT][4][64];  // the next pivot block, from the waves' quarters to their strips
+    } sh;
+    const int tpr = (m + 63) / 64;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    const int q = lane >> 4, r = lane & 15;
+    const int nb = min(INV_NB, m - k), kn = k + INV_NB;
+    // the next pivot block trades places with block 0 in the launch order (no next one: none)
+    const int dn = kn < m ? (kn / 64) * (tpr + 1) : 0;
+    const int t = (int)blockIdx.x == 0 ? dn : (int)blockIdx.x == dn ? 0 : (int)blockIdx.x;
+    const int row0 = (t / tpr) * 64 + 32 * (wave >> 1), col0 = (t % tpr) * 64 + 32 * (wave & 1);
+    const auto* Ab = gmem(Wa) + (long long)blockIdx.y * m * m;
+    auto* Bb = gmem(Wb) + (long long)blockIdx.y * m * m;
+    const auto* Mb = gmem(Mm) + (long long)blockIdx.y * m * INV_NB;
+    td4 acc[2][2];
+    if ((t % tpr) * 64 == k) {  // pivot columns
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int v = 0; v < 4; v++)
+                    acc[i][j][v] = Mb[(long long)min(row0 + 16 * i + 4 * v + q, m - 1) * INV_NB + col0 - k + 16 * j + r];
+    } else {
+        const bool pivot_rows = (t / tpr) * 64 == k;
+        const int c0 = min(col0 + r, m - 1), c1 = min(col0 + 16 + r, m - 1);
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const long long row = (long long)min(row0 + 16 * i + 4 * v + q, m - 1) * m;
+                const double x = Ab[row + c0], y = Ab[row + c1];
+                acc[i][0][v] = pivot_rows ? 0.0 : x;
+                acc[i][1][v] = pivot_rows ? 0.0 : y;
+            }
+        const auto* m0 = Mb + (long long)min(row0 + r, m - 1) * INV_NB;
+        const auto* m1 = Mb + (long long)min(row0 + 16 + r, m - 1) * INV_NB;
+#pragma unroll
+        for (int kb = 0; kb < INV_NB; kb += 16) {
+            const int k0 = kb + 4 * q;  // lane group q takes k = kb + 4q + s at step s
+            double a0[4], a1[4], b0[4], b1[4];
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                a0[s] = m0[k0 + s];
+                a1[s] = m1[k0 + s];
+                const auto* brow = Ab + (long long)(k + min(k0 + s, nb - 1)) * m;  // past nb: times a zero
+                b0[s] = brow[c0];
+                b1[s] = brow[c1];
+            }
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                acc[0][0] = mfma_f64(a0[s], b0[s], acc[0][0]);
+                acc[0][1] = mfma_f64(a0[s], b1[s], acc[0][1]);
+                acc[1][0] = mfma_f64(a1[s], b0[s], acc[1][0]);
+                acc[1][1] = mfma_f64(a1[s], b1[s], acc[1][1]);
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int row = row0 + 16 * i + 4 * v + q, col = col0 + 16 * j + r;
+                if (row < m && col < m) Bb[(long long)row * m + col] = acc[i][j][v];
+            }
+    if (kn >= m || blockIdx.x != 0) return;  // uniform per workgroup
+    const int nn = min(INV_NB, m - kn);
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) sh.blk[2 * (wave >> 1) + i][2 * (wave & 1) + j][v][lane] = acc[i][j][v];
+    __syncthreads();
+    td4 T[MT];
+#pragma unroll
+    for (int j = 0; j < MT; j++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const int row = 16 * wave + 4 * v + q, col = 16 * j + r;
+            const double x = sh.blk[wave][j][v][lane];
+            T[j][v] = (row < nn && col < nn) ? x : (row == col ? 1.0 : 0.0);
+        }
+    __syncthreads();
+    inv_pivot_block(T, nn, sh.inv, Pn + (long long)blockIdx.y * INV_NB * INV_NB, flag);
+}
+
+// ---------------------------------------------------------------------------------------
 // Merge assembly
 // ---------------------------------------------------------------------------------------
 // block (sa, sb) element (i, j) of a child DtN map (4n x 4n, WESN blocks of n)
@@ -1042,20 +1576,29 @@ __global__ void __launch_bounds__(256) tree_root_dirichlet_kernel(const double* 
     g[(long long)c * vrows + i] = r[e] / a[i];
 }
 
-// A = diag(a) + diag(b) T and rhs = r - b h (HPSAlgorithm.hpp:402-420); rhs is [rhs][m], h a
+// A = diag(a) + diag(b) T and rhs = r - b h (HPSAlgorithm.hpp:402-420), row-scaled; rhs is [rhs][m], h a
 // column of the arena (h + rhs * vrows) or null.
 __global__ void __launch_bounds__(256) tree_root_robin_kernel(const double* T, const double* a, const double* b, const double* r,
                                                               const double* h, double* A, double* rhs, int m, int k,
                                                               long long vrows) {
     const long long e = (long long)blockIdx.x * 256 + threadIdx.x;
     const long long nA = (long long)m * m;
+    // rows scaled by powers of two to diag(a / b) + T, which is definite up to row signs as T is (a
+    // positive a / b outwards), and Dirichlet rows (b = 0) to the size of T's diagonal: then
+    // the elimination in natural order meets no large multiplier
+    auto scale = [&](int i) {
+        auto fine = [](double x) { return fabs(x) > 1e-150 && fabs(x) < 1e150; };
+        const double t = T[(long long)i * m + i];
+        if (fine(b[i])) return ldexp(1.0, -ilogb(b[i]));
+        return b[i] == 0.0 && fine(a[i]) && fine(t) ? ldexp(1.0, ilogb(t) - ilogb(a[i])) : 1.0;
+    };
     if (e < nA) {
         const int i = (int)(e / m), j = (int)(e % m);
-        A[e] = b[i] * T[e] + (i == j ? a[i] : 0.0);
+        A[e] = scale(i) * (b[i] * T[e] + (i == j ? a[i] : 0.0));
     } else if (e < nA + (long long)m * k) {
         const long long t = e - nA;
         const int c = (int)(t / m), i = (int)(t % m);
-        rhs[t] = r[t] - b[i] * (h ? h[(long long)c * vrows + i] : 0.0);
+        rhs[t] = scale(i) * (r[t] - b[i] * (h ? h[(long long)c * vrows + i] : 0.0));
     }
 }
 
@@ -1235,6 +1778,48 @@ void run_gj_inverse(double* wa, double* xi, int m, int B, const GJWork& w, int* 
     a.Wa = cur; a.Wb = nxt; a.k = 0;
     EF_LAUNCH("gj_perm_kernel", gj_perm_kernel, dim3(B), dim3(256), s, a);
     EF_LAUNCH("gj_gather_kernel", gj_gather_kernel, dim3(blocks_for((long long)m * m), B), dim3(256), s, a);
+}
+
+size_t inv_work_doubles(int m, int B) {
+    return m <= INV_SMALL ? 0 : (size_t)B * ((size_t)m * m + (size_t)m * INV_NB + (size_t)INV_NB * INV_NB);
+}
+
+void run_inverse(double* wa, double* xi, int m, int B, double* work, int* flag, hipStream_t s) {
+    if (B <= 0) return;
+    if (m < 1 || m > GJ_MAXM)
+        throw EfError(EF_ERR_ARG, "interface system of order " + std::to_string(m) + " exceeds the inversion limit " +
+                                      std::to_string(GJ_MAXM));
+    const size_t mm = (size_t)m * m * B;
+    check_range(wa, mm * 8, "matrices to invert");
+    check_range(xi, mm * 8, "inverse output");
+    check_range(flag, sizeof(int), "inversion flag");
+    // up to 64 one wave holds the matrix (128 registers a lane), up to 128 a workgroup of eight
+    if (m <= 16)
+        EF_LAUNCH("inv_wave_kernel<1>", inv_wave_kernel<1>, dim3((B + 3) / 4), dim3(256), s, (const double*)wa, xi, m, B, flag);
+    else if (m <= 32)
+        EF_LAUNCH("inv_wave_kernel<2>", inv_wave_kernel<2>, dim3((B + 3) / 4), dim3(256), s, (const double*)wa, xi, m, B, flag);
+    else if (m <= 64)
+        EF_LAUNCH("inv_wave_kernel<4>", inv_wave_kernel<4>, dim3((B + 3) / 4), dim3(256), s, (const double*)wa, xi, m, B, flag);
+    else if (m <= INV_SMALL)
+        EF_LAUNCH("inv_small_kernel<8>", inv_small_kernel<8>, dim3(B), dim3(512), s, (const double*)wa, xi, m, flag);
+    else {
+        check_range(work, inv_work_doubles(m, B) * 8, "inversion work");
+        if (m % 4 != 0) throw EfError(EF_ERR_INTERNAL, "inversion of an order that is not a multiple of 4");
+        double* Mm = work + mm;
+        double* Pn = Mm + (size_t)B * m * INV_NB;
+        double* cur = wa;
+        double* nxt = work;
+        const int tpr = (m + 63) / 64;
+        EF_LAUNCH("inv_pivot_kernel", inv_pivot_kernel, dim3(B), dim3(256), s, (const double*)cur, Pn, m, flag);
+        for (int k = 0; k < m; k += INV_NB) {
+            double* out = (k + INV_NB >= m) ? xi : nxt;  // the last step writes the inverse where it belongs
+            EF_LAUNCH("inv_mult_kernel", inv_mult_kernel, dim3(tpr, B), dim3(512), s, (const double*)cur, Mm,
+                      (const double*)Pn, m, k, flag);
+            EF_LAUNCH("inv_update_kernel", inv_update_kernel, dim3(tpr * tpr, B), dim3(256), s, (const double*)cur, out,
+                      (const double*)Mm, Pn, m, k, flag);
+            std::swap(cur, nxt);
+        }
+    }
 }
 
 }  // namespace efk

@@ -146,6 +146,25 @@ __global__ void gj_perm_kernel(GJArgs a);
 __global__ void gj_gather_kernel(GJArgs a);
 
 // ---------------------------------------------------------------------------------------
+// Inversion of a batch of equally sized matrices by Gauss-Jordan in natural order (no row
+// exchanges): in registers, one workgroup per matrix, up to INV_SMALL; beyond it INV_NB columns
+// per step (mult, update) between two buffers.  A multiplier beyond INV_LMAX (or a NaN) sets the
+// flag: the result is then not to be used.  4 is three times the largest multiplier of the
+// definite systems measured (1.3) and keeps the growth of an indefinite one that passes small.
+// ---------------------------------------------------------------------------------------
+constexpr int INV_SMALL = 128;
+constexpr int INV_NB = 64;
+constexpr double INV_LMAX = 4.0;
+
+template <int MT>
+__global__ void inv_wave_kernel(const double* A, double* Ai, int m, int B, int* flag);
+template <int MT>
+__global__ void inv_small_kernel(const double* A, double* Ai, int m, int* flag);
+__global__ void inv_pivot_kernel(const double* A, double* Pn, int m, int* flag);
+__global__ void inv_mult_kernel(const double* A, double* Mm, const double* Pn, int m, int k, int* flag);
+__global__ void inv_update_kernel(const double* Wa, double* Wb, const double* Mm, double* Pn, int m, int k, int* flag);
+
+// ---------------------------------------------------------------------------------------
 // Merge assembly (createMatrixBlocks_ + mergeX_ + the block-diagonal part of mergeT_,
 // HPSAlgorithm.hpp:799-968, with the WESN order of reorderOperators_, :979-993): from the
 // four children's DtN maps (each 4n x 4n, coarsened), X (4n x 4n) into the inversion work
@@ -219,5 +238,11 @@ struct GJWork {
 size_t gj_work_doubles(int m, int B);  // doubles of wb + Pinv + Mm
 size_t gj_work_ints(int m, int B);     // ints of cand + src + ipiv + prow
 void run_gj_inverse(double* wa, double* xi, int m, int B, const GJWork& w, int* info, hipStream_t s);
+
+// Inversion in natural order of `B` matrices of order m held in wa (B x m x m, destroyed beyond
+// INV_SMALL); X^-1 into xi.  work: inv_work_doubles(m, B); *flag is set when a multiplier was too
+// large (never cleared here).
+size_t inv_work_doubles(int m, int B);
+void run_inverse(double* wa, double* xi, int m, int B, double* work, int* flag, hipStream_t s);
 
 }  // namespace efk
