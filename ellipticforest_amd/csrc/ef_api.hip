@@ -428,11 +428,16 @@ struct ef_mesh_s {
     // leaf classes
     std::vector<PatchCoef> classes_h;  // one per distinct (stencil, dx, dy)
     std::vector<int> leaf_class;       // per leaf
+    // leaves by cell size (dx, dy), the classes of constant coefficients; found once per mesh
+    std::vector<int> geom_class;
+    std::vector<std::pair<double, double>> geom_dxy;
+    bool geom_on_device = false;       // leaf_cls holds geom_class
     int tleaf_class0 = -1;
     DevBuf<PatchCoef> classes;
     DevBuf<int> leaf_cls;                  // per leaf, on the device
     DevBuf<long long> leaf_goff, leaf_hoff;  // vector-arena rows of each leaf's g and h
     DevBuf<LeafDesc> leafdesc;             // block-tridiagonal path
+    std::vector<double> mu_h;
     DevBuf<double> QA, QB, mu, dinv, leafT;  // fast-diagonalisation tables, leaf DtN
     // variable-coefficient leaves (block-tridiagonal path)
     bool variable = false;
@@ -449,6 +454,7 @@ struct ef_mesh_s {
     std::vector<GroupPlan> gplans;
     DevStore bstore;
     std::vector<const void*> plan_sig;  // arena and leaf-DtN addresses gplans was made for
+    std::vector<const void*> sweep_sig;  // every address the sweep plans and captured sweeps hold
     // vectors
     int kcap = 0;
     int k_up = 0;  // k of the last upwards call
@@ -459,6 +465,9 @@ struct ef_mesh_s {
     // root Robin work
     DevBuf<double> rootA, rootAi, rootgj, rootrhs;
     DevBuf<int> rootgji, rootinfo;
+    DevStore root_store;                 // descriptors of the product with the root system's inverse
+    GemmLaunch root_gemm;
+    std::array<const void*, 4> root_sig{};  // its addresses and k (in the last entry)
     // stage timers: event pairs for build, upwards, solve
     hipEvent_t ev[3][2] = {{nullptr, nullptr}, {nullptr, nullptr}, {nullptr, nullptr}};
     bool ev_recorded[3] = {false, false, false};
@@ -625,51 +634,65 @@ void setup_leaf_classes(ef_mesh_s* M, const ef_coeffs& c) {
         M->leafdesc.upload(ld, M->stream);
         return;
     }
-    std::map<std::vector<uint64_t>, int> seen;
-    auto bits = [](double v) { uint64_t u; std::memcpy(&u, &v, 8); return u; };
-    for (size_t li = 0; li < nl; li++) {
-        const NodeP& nd = P.nodes[P.leaves[li]];
-        const double dx = (nd.xu - nd.xl) / N, dy = (nd.yu - nd.yl) / N;
-        double cx, cy, lam;
-        if (c.solver_type == EF_SOLVER_FISHPACK) {
-            cx = 1.0 / (dx * dx); cy = 1.0 / (dy * dy); lam = c.lambda0;
-        } else if (c.cell == nullptr) {
-            cx = c.alpha0 * c.beta0 / (dx * dx); cy = c.alpha0 * c.beta0 / (dy * dy); lam = c.lambda0;
-        } else {
-            // per-cell samples constant over this leaf
-            const double* cc = c.cell + li * 6 * NN;
-            cx = cc[0] * cc[NN] / (dx * dx); cy = cc[0] * cc[NN] / (dy * dy); lam = cc[5 * NN];
+    auto coef = [&](double cx, double cy, double lam, double dx, double dy) {
+        PatchCoef k;
+        k.cx = cx; k.cy = cy; k.lam = lam; k.dx = dx; k.dy = dy;
+        M->classes_h.push_back(k);
+    };
+    if (c.solver_type == EF_SOLVER_FISHPACK || c.cell == nullptr) {
+        // one coefficient set: a class per cell size
+        if (M->geom_class.empty()) {
+            std::map<std::pair<double, double>, int> seen;
+            for (size_t li = 0; li < nl; li++) {
+                const NodeP& nd = P.nodes[P.leaves[li]];
+                const auto d = std::make_pair((nd.xu - nd.xl) / N, (nd.yu - nd.yl) / N);
+                const auto it = seen.emplace(d, (int)seen.size());
+                if (it.second) M->geom_dxy.push_back(d);
+                M->geom_class.push_back(it.first->second);
+            }
         }
-        std::vector<uint64_t> key = {bits(cx), bits(cy), bits(lam), bits(dx), bits(dy)};
-        auto it = seen.find(key);
-        int id;
-        if (it == seen.end()) {
-            id = (int)M->classes_h.size();
-            seen[key] = id;
-            PatchCoef k;
-            k.cx = cx; k.cy = cy; k.lam = lam; k.dx = dx; k.dy = dy;
-            M->classes_h.push_back(k);
-        } else id = it->second;
-        M->leaf_class[li] = id;
+        M->leaf_class = M->geom_class;
+        const double ab = c.solver_type == EF_SOLVER_FISHPACK ? 1.0 : c.alpha0 * c.beta0;
+        for (const auto& d : M->geom_dxy)
+            coef(ab / (d.first * d.first), ab / (d.second * d.second), c.lambda0, d.first, d.second);
+    } else {
+        // per-cell samples constant over each leaf
+        std::map<std::vector<uint64_t>, int> seen;
+        auto bits = [](double v) { uint64_t u; std::memcpy(&u, &v, 8); return u; };
+        for (size_t li = 0; li < nl; li++) {
+            const NodeP& nd = P.nodes[P.leaves[li]];
+            const double dx = (nd.xu - nd.xl) / N, dy = (nd.yu - nd.yl) / N;
+            const double* cc = c.cell + li * 6 * NN;
+            const double cx = cc[0] * cc[NN] / (dx * dx), cy = cc[0] * cc[NN] / (dy * dy), lam = cc[5 * NN];
+            const auto it = seen.emplace(std::vector<uint64_t>{bits(cx), bits(cy), bits(lam), bits(dx), bits(dy)}, (int)seen.size());
+            if (it.second) coef(cx, cy, lam, dx, dy);
+            M->leaf_class[li] = it.first->second;
+        }
+        M->geom_on_device = false;
     }
     M->tleaf_class0 = M->leaf_class[0];
     const int ncls = (int)M->classes_h.size();
     M->leafT.ensure((size_t)ncls * 16 * NN);
     M->classes.upload(M->classes_h, M->stream);
-    M->leaf_cls.upload(M->leaf_class, M->stream);
-    std::vector<long long> goff(4 * nl), hoff(nl);
-    for (size_t li = 0; li < nl; li++) {
-        for (int sd = 0; sd < 4; sd++) goff[4 * li + sd] = P.nodes[P.leaves[li]].gsrc[sd];
-        hoff[li] = P.nodes[P.leaves[li]].h_off;
+    const bool geom = c.solver_type == EF_SOLVER_FISHPACK || c.cell == nullptr;
+    if (!geom || !M->geom_on_device) M->leaf_cls.upload(M->leaf_class, M->stream);
+    M->geom_on_device = geom;
+    if (!M->QA.p) {  // what depends on the mesh alone
+        std::vector<long long> goff(4 * nl), hoff(nl);
+        for (size_t li = 0; li < nl; li++) {
+            for (int sd = 0; sd < 4; sd++) goff[4 * li + sd] = P.nodes[P.leaves[li]].gsrc[sd];
+            hoff[li] = P.nodes[P.leaves[li]].h_off;
+        }
+        M->leaf_goff.upload(goff, M->stream);
+        M->leaf_hoff.upload(hoff, M->stream);
+        std::vector<double> QA, QB;
+        patch_fd_tables(N, N <= 16 ? 1 : 2, QA, QB, M->mu_h);
+        M->QB.upload(QB, M->stream);
+        M->mu.upload(M->mu_h, M->stream);
+        M->QA.upload(QA, M->stream);
     }
-    M->leaf_goff.upload(goff, M->stream);
-    M->leaf_hoff.upload(hoff, M->stream);
-    std::vector<double> QA, QB, mu, dinv;
-    patch_fd_tables(N, N <= 16 ? 1 : 2, QA, QB, mu);
-    patch_fd_dinv(N, N <= 16 ? 1 : 2, mu, M->classes_h, dinv);
-    M->QA.upload(QA, M->stream);
-    M->QB.upload(QB, M->stream);
-    M->mu.upload(mu, M->stream);
+    std::vector<double> dinv;
+    patch_fd_dinv(N, N <= 16 ? 1 : 2, M->mu_h, M->classes_h, dinv);
     M->dinv.upload(dinv, M->stream);
 }
 
@@ -840,7 +863,6 @@ void do_build(ef_mesh_s* M, const ef_coeffs& c) {
     hipStream_t s = M->stream;
     const int N = P.N;
     check_tree_kernels();
-    clear_graphs(M);  // captured sweeps read the operator arenas reallocated below
     M->solver_type = c.solver_type;
     setup_leaf_classes(M, c);
     // arenas and work (kept across builds of the mesh: their sizes depend on the tree only)
@@ -859,6 +881,18 @@ void do_build(ef_mesh_s* M, const ef_coeffs& c) {
         M->plan_sig.clear();
         plan_build(M);
         M->plan_sig = sig;
+    }
+    // sweep plans and captured sweeps hold addresses, not values: a build that moved none of them
+    // (new coefficients on a mesh that was built before) keeps both.  Planning 1,937 merges and
+    // capturing their sweeps again took 8 of the 11 host milliseconds of such a build
+    const void* leaf_addr[] = {M->classes.p, M->leaf_cls.p, M->leaf_goff.p, M->leaf_hoff.p, M->leafdesc.p, M->QA.p,
+                               M->QB.p, M->mu.p, M->dinv.p, (const void*)(intptr_t)(1 + M->variable + 2 * M->packed)};
+    sig.insert(sig.end(), std::begin(leaf_addr), std::end(leaf_addr));
+    if (sig != M->sweep_sig) {
+        M->sweep_sig.clear();
+        clear_graphs(M);
+        M->sweeps.clear();
+        M->sweep_sig = std::move(sig);
     }
     if (M->variable) {
         // block-tridiagonal factors, then the DtN of every leaf (buildD2N) in chunks of leaves
@@ -1440,16 +1474,21 @@ void do_solve_once(ef_mesh_s* M, const double* f_dev, const double* r_dev, const
             efk::copy_d2h(info, M->rootinfo.p, sizeof(int), s);
             if (info[0]) throw EfError(EF_ERR_SINGULAR, "zero pivot in the root boundary system");
         }
-        TreeGemm p{};
-        p.A0 = M->rootAi.p; p.lda0 = m; p.K0 = m; p.alpha0 = 1.0;
-        p.B0 = M->rootrhs.p; p.ldb0 = 1; p.bcs = m;
-        p.D = V + root.g_off; p.ldd = 1; p.dcs = (int)P.vec_rows;
-        p.M = m; p.N = k;
-        DevStore tmp;
-        GemmLaunch g = plan_gemm(std::vector<TreeGemm>{p}, k <= 16 ? 1 : 2, tmp, s);
-        tmp.flush(s);
-        run_gemm(g, s);
-        EF_HIP(hipStreamSynchronize(s));  // the launch's descriptors are freed here
+        const std::array<const void*, 4> rsig = {M->rootAi.p, M->rootrhs.p, V, (const void*)(intptr_t)k};
+        if (rsig != M->root_sig) {
+            M->root_sig = {};
+            EF_HIP(hipStreamSynchronize(s));  // an earlier solve may still read the descriptors
+            M->root_store.clear();
+            TreeGemm p{};
+            p.A0 = M->rootAi.p; p.lda0 = m; p.K0 = m; p.alpha0 = 1.0;
+            p.B0 = M->rootrhs.p; p.ldb0 = 1; p.bcs = m;
+            p.D = V + root.g_off; p.ldd = 1; p.dcs = (int)P.vec_rows;
+            p.M = m; p.N = k;
+            M->root_gemm = plan_gemm(std::vector<TreeGemm>{p}, k <= 16 ? 1 : 2, M->root_store, s);
+            M->root_store.flush(s);
+            M->root_sig = rsig;
+        }
+        run_gemm(M->root_gemm, s);
     }
     downward();
 }
@@ -1688,7 +1727,6 @@ int ef_build(ef_mesh mesh, const ef_coeffs* coeffs, int precision) {
     EF_HIP(hipSetDevice(mesh->ctx->device));
     if (precision == EF_PRECISION_MIXED) setup_mixed(mesh);
     mesh->built = false;
-    mesh->sweeps.clear();
     mesh->k_up = 0;
     mesh->precision = precision;
     stage_begin(mesh, 0);
