@@ -763,7 +763,7 @@ __device__ inline double wave_half_sum(double x) {
     return __hiloint2double((int)sh[0], (int)sl[0]) + __hiloint2double((int)sh[1], (int)sl[1]);
 }
 
-// One wave per (leaf, rhs) as bt_solve_wave_kernel, on the packed blocks.  The 2 NT - 1 block
+// One wave per (leaf, rhs) as bt_solve_wave_kernel, on the packed blocks (N = 8).  The 2 NT - 1 block
 // steps (forward i = 0 .. NT-1, then backward i = NT-2 .. 0) form one sequence; while step s
 // computes on block s in one of the wave's two LDS slots, block s + 1 waits in the other and
 // block s + 2 is on its way into registers, so the backward sweep's first blocks arrive during
@@ -923,10 +923,186 @@ bt_solve_sym_kernel(const LeafDesc* leaves, int nleaves, int k, int mode, const 
 
 template __global__ void bt_solve_sym_kernel<8>(const LeafDesc*, int, int, int, const double*, int, const double*,
                                                 double*, double*, long long);
-template __global__ void bt_solve_sym_kernel<16>(const LeafDesc*, int, int, int, const double*, int, const double*,
-                                                 double*, double*, long long);
-template __global__ void bt_solve_sym_kernel<32>(const LeafDesc*, int, int, int, const double*, int, const double*,
-                                                 double*, double*, long long);
+
+// The same substitution for N = NT in {16, 32} on v_mfma_f64_4x4x4f64, one wave per leaf and four
+// right-hand sides (`chunks` of them; the waves of one leaf lie side by side and share its packed
+// blocks' reads in the caches): reading the blocks (N^2 (N + 1) / 2 entries, forward and backward) is
+// what bounds the solve.  One wave per right-hand side read them k times: 4,096 leaves of 32 x 32
+// cells at k = 4 took 889 us (Neumann data) and 977 us (solve), so 330 us each; at k = 1 it is the
+// memory rate either way (270 us, 4.7 TB/s).  Two or four groups of four per wave (blocks read once
+// for 16) were 10 % faster at 1,024 leaves and k = 16, and up to twice as slow on meshes whose leaves
+// do not fill the chip.
+// The instruction multiplies four 4 x 4 blocks: lane 16 k + 4 b + i holds A_b(i, k), lane 16 k + 4 b + j
+// B_b(k, j), lane 16 i + 4 b + j D_b(i, j).  Block b takes rows 16 h + 4 b .. + 3 of the block row (h <
+// NT / 16) and the four columns are four right-hand sides; every block of an operand B is the
+// same, read from LDS where the lanes put the vector.  A column's sums do not depend on the others.
+constexpr int BT_RHS = 4;  // right-hand sides per wave
+template <int NT>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8)))
+bt_solve_mfma_kernel(const LeafDesc* leaves, int nleaves, int k, int mode, const double* f, int f_zero,
+                     const double* garena, double* harena, double* zbuf, long long vcs) {
+    using PK = BtPack<NT>;
+    constexpr int NN = NT * NT, R = PK::R, STEPS = 2 * NT - 1, H = NT / 16, KS = NT / 4;
+    constexpr int PD = 4;  // steps a load is issued ahead
+    static_assert(NT % PD == 0, "the sweeps turn on a whole round of the load ring");
+    __shared__ double sp_all[4][2][PK::LSIZE];
+    __shared__ double tv_all[4][NT * 4 + 16];
+    __shared__ double eg_all[4][4][NT * 4];  // boundary forcing of the four sides' cells
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int chunks = (k + BT_RHS - 1) / BT_RHS;
+    const long long items = (long long)nleaves * chunks;
+    const int qi = lane >> 4, b = (lane >> 2) & 3, j = lane & 3;  // qi: A's k, D's row in its block; j: A's row, column
+    double* tv = tv_all[wave];
+    double (*eg)[NT * 4] = eg_all[wave];
+    int row[H];
+#pragma unroll
+    for (int h = 0; h < H; h++) row[h] = 16 * h + 4 * b + qi;
+    // k = 4 ks + qi of the products is column ccol + ks of the block: the four lane groups a quarter of the
+    // row apart, the first two half a row, so that the 16 rows they read lie in different LDS banks
+    const int ccol = (NT / 2) * (qi & 1) + (NT / 4) * (qi >> 1);
+    auto tvi = [](int r) { return r * 4 + (r / (NT / 4)) * 4; };  // row r of the vector in tv
+    // where this lane's A operands lie in a staged block: S(16 h + 4 b + j, ccol + ks), upper triangle
+    int at[H][KS];
+#pragma unroll
+    for (int h = 0; h < H; h++)
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+            const int r = 16 * h + 4 * b + j, c = ccol + ks;
+            at[h][ks] = PK::lds(min(r, c), max(r, c));
+        }
+    auto blk = [](int s) { return s < NT ? s : 2 * NT - 2 - s; };
+    // the loop's bounds are uniform per wave; no barrier between waves
+    for (long long item = (long long)blockIdx.x * 4 + wave; item < items; item += (long long)gridDim.x * 4) {
+        const int leaf = (int)(item / chunks), rhs0 = (int)(item % chunks) * BT_RHS;
+        const LeafDesc L = leaves[leaf];
+        const auto* cWv = gmem((const double*)L.stencil);
+        const auto* SP = gmem((const double*)L.SinvP);
+        // this lane's right-hand side (past the last one: the last, not stored)
+        const int rhs = min(rhs0 + j, k - 1);
+        const bool live = rhs0 + j < k;
+        const long long vo = ((long long)rhs * nleaves + leaf) * NN;  // the leaf in f and zbuf
+        const auto* g = gmem(garena) + (long long)rhs * vcs;          // (not read without g)
+        if (mode != 0) {
+            // -2 c_side g_side on the edge cells (ghost 2 g - u, FiniteVolumeSolver.cpp:100-184)
+#pragma unroll
+            for (int h = 0; h < H; h++) {
+                const int t = row[h];
+                eg[W][t * 4 + j] = -2.0 * cWv[t] * g[L.gs[W] + t];
+                eg[E][t * 4 + j] = -2.0 * cWv[NN + (NT - 1) * NT + t] * g[L.gs[E] + t];
+                eg[S][t * 4 + j] = -2.0 * cWv[2 * NN + t * NT] * g[L.gs[S] + t];
+                eg[N][t * 4 + j] = -2.0 * cWv[3 * NN + t * NT + NT - 1] * g[L.gs[N] + t];
+            }
+        }
+        auto load = [&](int s, double (&Rr)[R]) {
+            const auto* src = SP + (long long)blk(s) * L.pstride;
+#pragma unroll
+            for (int r = 0; r < R; r++) Rr[r] = src[min(lane + 64 * r, PK::NP - 1)];
+        };
+        auto stage = [&](const double (&Rr)[R], int slot) {
+            double* sp = sp_all[wave][slot];
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                const int e = lane + 64 * r;
+                if (e < PK::NP) sp[e + e / PK::PAIR] = Rr[r];
+            }
+        };
+        // step s's inputs from memory: f and cW of block row i, or z and cE of it
+        auto inputs = [&](int s, double (&x)[H], double (&c)[H]) {
+            const int i = blk(s);
+            const bool fwd = s < NT;
+            const auto* v = gmem(fwd && !f_zero ? f : (const double*)zbuf) + vo;
+#pragma unroll
+            for (int h = 0; h < H; h++) {
+                c[h] = cWv[(fwd ? 0 : NN) + i * NT + row[h]];
+                x[h] = v[i * NT + row[h]];
+            }
+        };
+        const double sx = 2.0 / L.dx, sy = 2.0 / L.dy;
+        // Neumann data of block row i's edge cells (mapD2N, FiniteVolumeSolver.cpp:296-353)
+        auto emit = [&](int i, int h, double x) {
+            if (!live) return;
+            auto* hv = gmem(harena) + (long long)rhs * vcs + L.h_off;
+            auto gv = [&](long long side, int t) { return mode != 0 ? g[side + t] : 0.0; };
+            if (i == 0) hv[W * NT + row[h]] = sx * (x - gv(L.gs[W], row[h]));
+            if (i == NT - 1) hv[E * NT + row[h]] = -sx * (x - gv(L.gs[E], row[h]));
+            if (row[h] == 0) hv[S * NT + i] = sy * (x - gv(L.gs[S], i));
+            if (row[h] == NT - 1) hv[N * NT + i] = -sy * (x - gv(L.gs[N], i));
+        };
+        // A ring of PD steps' loads: what step s reads was issued PD steps before.  (Waits count loads
+        // in issue order: inputs loaded one step ahead made every step wait for the blocks as well.)
+        double Rr[PD][R], xr[PD][H], cr[PD][H], zk[PD][H];
+        load(0, Rr[0]);
+        load(1, Rr[1]);
+        stage(Rr[0], 0);
+        stage(Rr[1], 1);
+#pragma unroll
+        for (int u = 0; u < PD; u++) {
+            inputs(u, xr[u], cr[u]);
+            load(2 + u, Rr[u]);
+        }
+        double z[H];  // the last row of the sweep
+#pragma unroll
+        for (int h = 0; h < H; h++) z[h] = 0.0;
+        __builtin_amdgcn_wave_barrier();
+        for (int s0 = 0; s0 < STEPS; s0 += PD) {
+#pragma unroll
+            for (int u = 0; u < PD; u++) {
+                const int s = s0 + u;
+                if (s >= STEPS) break;
+                const bool fwd = s < NT;
+                const int i = blk(s);
+                const double* sp = sp_all[wave][s & 1];
+                // forward z_i = Sinv_i (b_i - cW_i .* z_{i-1}); backward x_i = z_i - Sinv_i (cE_i .* x_{i+1})
+                double acc[H];
+#pragma unroll
+                for (int h = 0; h < H; h++) {
+                    double x = fwd && f_zero ? 0.0 : xr[u][h];
+                    // the first backward rows were still in registers when their loads were due
+                    if (u < PD - 1 && s0 == NT) x = zk[PD - 2 - u][h];
+                    if (fwd && mode != 0) {
+                        if (i == 0) x += eg[W][row[h] * 4 + j];
+                        if (i == NT - 1) x += eg[E][row[h] * 4 + j];
+                        const double es = eg[S][i * 4 + j], en = eg[N][i * 4 + j];
+                        x += (row[h] == 0) ? es : 0.0;
+                        x += (row[h] == NT - 1) ? en : 0.0;
+                    }
+                    const double cz = s > 0 ? cr[u][h] * z[h] : 0.0;
+                    acc[h] = fwd ? 0.0 : x;
+                    tv[tvi(row[h]) + j] = fwd ? x - cz : -cz;
+                }
+                if (s + PD < STEPS) inputs(s + PD, xr[u], cr[u]);
+                __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                for (int ks = 0; ks < KS; ks++) {
+                    const double B = tv[tvi(ccol + ks) + j];
+#pragma unroll
+                    for (int h = 0; h < H; h++) acc[h] = __builtin_amdgcn_mfma_f64_4x4x4f64(sp[at[h][ks]], B, acc[h], 0, 0, 0);
+                }
+                __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                for (int h = 0; h < H; h++) {
+                    z[h] = acc[h];
+                    if (fwd) zk[u][h] = acc[h];
+                    // z_{N-1} is x_{N-1}; each lane reads back only what it wrote
+                    const bool out = s >= NT - 1;
+                    if (live && (!out || mode == 1)) gmem(zbuf)[vo + i * NT + row[h]] = acc[h];
+                    if (out && mode != 1) emit(i, h, acc[h]);
+                }
+                // slot s & 1 is free once step s has read it (the wave's LDS accesses run in order)
+                if (s + 2 < STEPS) {
+                    stage(Rr[u], s & 1);
+                    if (s + 2 + PD < STEPS) load(s + 2 + PD, Rr[u]);
+                }
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
+template __global__ void bt_solve_mfma_kernel<16>(const LeafDesc*, int, int, int, const double*, int, const double*,
+                                                  double*, double*, long long);
+template __global__ void bt_solve_mfma_kernel<32>(const LeafDesc*, int, int, int, const double*, int, const double*,
+                                                  double*, double*, long long);
 
 void launch_bt_solve(const LeafDesc* leaves, int Nn, int nleaves, int k, int mode, const double* f, int f_zero,
                      const double* garena, double* harena, double* u, hipStream_t s, bool packed, double* zwork,
@@ -937,12 +1113,17 @@ void launch_bt_solve(const LeafDesc* leaves, int Nn, int nleaves, int k, int mod
     if (packed && Nn == 8)
         hipLaunchKernelGGL(bt_solve_sym_kernel<8>, dim3(blocks), dim3(256), 0, s, leaves, nleaves, k, mode, f, f_zero,
                            garena, harena, zbuf, vcs);
-    else if (packed && Nn == 16)
-        hipLaunchKernelGGL(bt_solve_sym_kernel<16>, dim3(blocks), dim3(256), 0, s, leaves, nleaves, k, mode, f,
-                           f_zero, garena, harena, zbuf, vcs);
-    else if (packed && Nn == 32)
-        hipLaunchKernelGGL(bt_solve_sym_kernel<32>, dim3(blocks), dim3(256), 0, s, leaves, nleaves, k, mode, f,
-                           f_zero, garena, harena, zbuf, vcs);
+    else if (packed && (Nn == 16 || Nn == 32)) {
+        // two workgroups per CU are resident; their waves stride over (leaf, four right-hand sides)
+        const long long items = (long long)nleaves * ((k + BT_RHS - 1) / BT_RHS);
+        const unsigned wg = (unsigned)std::min<long long>(512, (items + 3) / 4);
+        if (Nn == 16)
+            hipLaunchKernelGGL(bt_solve_mfma_kernel<16>, dim3(wg), dim3(256), 0, s, leaves, nleaves, k, mode, f, f_zero,
+                               garena, harena, zbuf, vcs);
+        else
+            hipLaunchKernelGGL(bt_solve_mfma_kernel<32>, dim3(wg), dim3(256), 0, s, leaves, nleaves, k, mode, f, f_zero,
+                               garena, harena, zbuf, vcs);
+    }
     else if (Nn == 8)
         hipLaunchKernelGGL(bt_solve_wave_kernel<8>, dim3(blocks), dim3(256), 0, s, leaves, nleaves, k, mode, f, f_zero,
                            garena, harena, u, vcs);

@@ -27,11 +27,14 @@ __global__ void bt_solve_wave_kernel(const LeafDesc* leaves, int nleaves, int k,
 template <int NT>
 __global__ void bt_solve_sym_kernel(const LeafDesc* leaves, int nleaves, int k, int mode, const double* f,
                                     int f_zero, const double* garena, double* harena, double* zbuf, long long vcs);
+template <int NT>
+__global__ void bt_solve_mfma_kernel(const LeafDesc* leaves, int nleaves, int k, int mode, const double* f,
+                                     int f_zero, const double* garena, double* harena, double* zbuf, long long vcs);
 __global__ void bt_pack_kernel(const LeafDesc* leaves, int nleaves, int Nn);
 // Leaf solves with variable coefficients: one wave per (leaf, rhs) for N in {8, 16, 32},
 // the workgroup-per-leaf kernel otherwise.  Modes as bt_solve_kernel.  With `packed`, every
 // leaf's SinvP holds its packed symmetric inverse pivot blocks (bt_pack_kernel), which the
-// kernel for N in {8, 16, 32} reads instead of Sinv; in modes 0 and 2 it needs zwork,
+// kernels for N in {8, 16, 32} read instead of Sinv (16 and 32: once for four right-hand sides); in modes 0 and 2 it needs zwork,
 // nleaves * k * N * N doubles of work space.  Boundary data and Neumann data of leaf L and
 // right-hand side c: garena / harena + c * vcs + L.g_off / L.h_off, 4N consecutive doubles.
 void launch_bt_solve(const LeafDesc* leaves, int Nn, int nleaves, int k, int mode, const double* f, int f_zero,

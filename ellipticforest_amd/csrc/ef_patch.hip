@@ -359,29 +359,23 @@ void record_end(ef_patches_s* p) {
     p->ev_recorded = true;
 }
 
-// Block-tridiagonal path, one right-hand side per launch ([patch][...] layouts with k = 1).
-// vz: work space of the packed Neumann maps, P N^2 doubles (null: the batch's own, grown as needed).
+// Block-tridiagonal path: launches of up to 16 right-hand sides (the packed Neumann maps' work grows
+// with them), [rhs][patch][...] layouts throughout.
+// vz: work space of the packed Neumann maps, P N^2 doubles, one right-hand side per launch (null: the
+// batch's own, grown as needed).
 void launch_bt(ef_patches_s* p, int op, const double* g, const double* f, double* out, int nrhs, double* vz = nullptr) {
     const long long NN = (long long)p->N * p->N, B4 = 4LL * p->N;
+    if (op == PATCH_OP_SOLVE && g == nullptr) throw EfError(EF_ERR_ARG, "boundary data g is required");
+    const int mode = op == PATCH_OP_SOLVE ? 1 : g ? 2 : 0;
+    const int step = vz ? 1 : 16;
     if (p->packed && op == PATCH_OP_MAP_D2N && !vz) {
-        p->vz.ensure((size_t)p->P * NN);
+        p->vz.ensure((size_t)p->P * NN * std::min(nrhs, step));
         vz = p->vz.p;
     }
-    if (op == PATCH_OP_MAP_D2N && g == nullptr) {
-        for (int c = 0; c < nrhs; c++) {
-            launch_bt_solve(p->leafdesc.p, p->N, p->P, 1, 0, f ? f + c * p->P * NN : nullptr, f ? 0 : 1,
-                            (const double*)nullptr, out + c * p->P * B4, (double*)nullptr, p->stream, p->packed,
-                            vz);
-            EF_LAUNCH_CHECK();
-        }
-        return;
-    }
-    if (g == nullptr) throw EfError(EF_ERR_ARG, "boundary data g is required");
-    const int mode = (op == PATCH_OP_SOLVE) ? 1 : 2;
-    for (int c = 0; c < nrhs; c++) {
-        launch_bt_solve(p->leafdesc.p, p->N, p->P, 1, mode, f ? f + c * p->P * NN : nullptr, f ? 0 : 1,
-                        g + c * p->P * B4, mode == 2 ? out + c * p->P * B4 : (double*)nullptr,
-                        mode == 1 ? out + c * p->P * NN : (double*)nullptr, p->stream, p->packed, vz);
+    for (int c = 0; c < nrhs; c += step) {
+        launch_bt_solve(p->leafdesc.p, p->N, p->P, std::min(step, nrhs - c), mode, f ? f + c * p->P * NN : nullptr, f ? 0 : 1,
+                        g ? g + c * p->P * B4 : (const double*)nullptr, mode == 1 ? (double*)nullptr : out + c * p->P * B4,
+                        mode == 1 ? out + c * p->P * NN : (double*)nullptr, p->stream, p->packed, vz, p->P * B4);
         EF_LAUNCH_CHECK();
     }
 }

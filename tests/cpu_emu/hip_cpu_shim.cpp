@@ -152,6 +152,19 @@ emu_d4 emu_mfma_f64(double a, double b, emu_d4 c, int, int, int) {
     return out;
 }
 
+// four 4 x 4 blocks b: lane 16 k + 4 b + i holds A(i, k), lane 16 k + 4 b + j B(k, j), lane 16 i + 4 b + j D(i, j)
+double emu_mfma_f64_4x4x4(double a, double b, double c, int, int, int) {
+    const int t = threadIdx.x, w = t / 64 * 64, l = t % 64;
+    const int p = g_par;
+    g_par ^= 1;
+    g_mfma_a[p][t] = a;
+    g_mfma_b[p][t] = b;
+    emu_wave_sync();
+    const int i = l / 16, blk = l / 4 % 4, j = l % 4;
+    for (int k = 0; k < 4; k++) c += g_mfma_a[p][w + 16 * k + 4 * blk + i] * g_mfma_b[p][w + 16 * k + 4 * blk + j];
+    return c;
+}
+
 emu_f4 emu_mfma_f32(float a, float b, emu_f4 c, int, int, int) {
     const int t = threadIdx.x, w = t / 64 * 64, l = t % 64;
     const int p = g_par;
