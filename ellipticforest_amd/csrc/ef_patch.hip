@@ -252,24 +252,7 @@ void launch_fd(ef_patches_s* p, int op, const double* g, const double* f, double
     efk::launch_patch_fd(a, p->NB, p->max_blocks, p->stream);
 }
 
-// Large patches: chunks of items through fold, four GEMMs, scaling and the output step.
-void launch_gemm_strided(const GemmStridedArgs& g, hipStream_t s) {
-    const long long blocks32 = (long long)((g.M + 31) / 32) * ((g.N + 31) / 32);  // one wave each
-    const dim3 grid((unsigned)((blocks32 + 3) / 4), (unsigned)g.batch), block(256);
-    // an operand is read as 32-byte vectors along k when it is contiguous along k and every
-    // row / column it starts from is 32-byte aligned
-    auto aligned = [](const double* x, long long s0, long long s1) {
-        return ((uintptr_t)x % 32 == 0) && s0 % 4 == 0 && s1 % 4 == 0;
-    };
-    const bool ak = g.ca == 1 && aligned(g.A, g.sa, g.ra);
-    const bool bk = g.rb == 1 && aligned(g.B, g.sb, g.cb);
-    if (ak && bk) hipLaunchKernelGGL((gemm_strided_f64_kernel<true, true>), grid, block, 0, s, g);
-    else if (ak) hipLaunchKernelGGL((gemm_strided_f64_kernel<true, false>), grid, block, 0, s, g);
-    else if (bk) hipLaunchKernelGGL((gemm_strided_f64_kernel<false, true>), grid, block, 0, s, g);
-    else hipLaunchKernelGGL((gemm_strided_f64_kernel<false, false>), grid, block, 0, s, g);
-    EF_LAUNCH_CHECK();
-}
-
+// Large patches: chunks of items through the four products and, for Neumann data, the edge cells.
 // W1, W2: work buffers of at least wcap doubles each (null: the batch's own, grown as needed).
 // Items are independent, so the chunking does not change any result.
 void launch_large(ef_patches_s* p, int op, const double* g, const double* f, double* out, int nrhs, int patch0 = 0,
@@ -287,6 +270,8 @@ void launch_large(ef_patches_s* p, int op, const double* g, const double* f, dou
         W1 = p->W1.p;
         W2 = p->W2.p;
     }
+    if (((uintptr_t)W1 | (uintptr_t)W2 | (uintptr_t)p->Qp.p) & 15)
+        throw EfError(EF_ERR_INTERNAL, "large-patch work buffers are not 16-byte aligned");
     for (long long first = 0; first < total; first += chunk) {
         const int items = (int)std::min(chunk, total - first);
         PatchLargeArgs a{};
@@ -301,38 +286,23 @@ void launch_large(ef_patches_s* p, int op, const double* g, const double* f, dou
         a.mu = p->mu.p;
         a.f = f;
         a.g = g;
-        a.work = W1;
+        a.Q = p->Qp.p;
+        a.W1 = W1;
+        a.W2 = W2;
         a.out = out;
         a.item0 = (op == PATCH_OP_DTN) ? 0 : first;
-        hipLaunchKernelGGL(patch_large_fold_kernel, dim3(blocks_for(items * per)), dim3(256), 0, p->stream, a);
+        const int tn = (Np + 31) / 32;
+        const dim3 grid((unsigned)(tn * tn), (unsigned)items), block(256);
+        hipLaunchKernelGGL(patch_large_gemm_kernel<0>, grid, block, 0, p->stream, a);
         EF_LAUNCH_CHECK();
-        GemmStridedArgs m{};
-        m.M = m.N = m.K = Np;
-        m.batch = items;
-        // W2 = Q^T W1
-        m.A = p->Qp.p; m.sa = 0; m.ra = 1; m.ca = Np;
-        m.B = W1; m.sb = per; m.rb = Np; m.cb = 1;
-        m.C = W2; m.sc = per; m.rc = Np; m.cc = 1;
-        launch_gemm_strided(m, p->stream);
-        // W1 = W2 Q
-        m.A = W2; m.sa = per; m.ra = Np; m.ca = 1;
-        m.B = p->Qp.p; m.sb = 0; m.rb = Np; m.cb = 1;
-        m.C = W1;
-        launch_gemm_strided(m, p->stream);
-        hipLaunchKernelGGL(patch_large_scale_kernel, dim3(blocks_for(items * per)), dim3(256), 0, p->stream, a);
+        hipLaunchKernelGGL(patch_large_gemm_kernel<1>, grid, block, 0, p->stream, a);
         EF_LAUNCH_CHECK();
-        // W2 = Q W1
-        m.A = p->Qp.p; m.sa = 0; m.ra = Np; m.ca = 1;
-        m.B = W1; m.sb = per; m.rb = Np; m.cb = 1;
-        m.C = W2;
-        launch_gemm_strided(m, p->stream);
-        // W1 = W2 Q^T
-        m.A = W2; m.sa = per; m.ra = Np; m.ca = 1;
-        m.B = p->Qp.p; m.sb = 0; m.rb = 1; m.cb = Np;
-        m.C = W1;
-        launch_gemm_strided(m, p->stream);
-        const long long nout = (op == PATCH_OP_SOLVE) ? (long long)items * N * N : (long long)items * 4 * N;
-        hipLaunchKernelGGL(patch_large_out_kernel, dim3(blocks_for(nout)), dim3(256), 0, p->stream, a);
+        hipLaunchKernelGGL(patch_large_gemm_kernel<2>, grid, block, 0, p->stream, a);
+        EF_LAUNCH_CHECK();
+        hipLaunchKernelGGL(patch_large_gemm_kernel<3>, grid, block, 0, p->stream, a);
+        EF_LAUNCH_CHECK();
+        if (op == PATCH_OP_SOLVE) continue;
+        hipLaunchKernelGGL(patch_large_out_kernel, dim3(blocks_for((long long)items * 4 * N)), dim3(256), 0, p->stream, a);
         EF_LAUNCH_CHECK();
     }
 }
