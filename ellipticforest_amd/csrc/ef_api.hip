@@ -810,8 +810,10 @@ void plan_build(ef_mesh_s* M) {
 
 void stage_begin(ef_mesh_s* M, int st) {
     if (!M->ev[st][0]) {
-        EF_HIP(hipEventCreate(&M->ev[st][0]));
-        EF_HIP(hipEventCreate(&M->ev[st][1]));
+        // timing only: without the system-scope release of a default event, which costs the stream 4 us
+        // a record against 2
+        EF_HIP(hipEventCreateWithFlags(&M->ev[st][0], hipEventDisableSystemFence));
+        EF_HIP(hipEventCreateWithFlags(&M->ev[st][1], hipEventDisableSystemFence));
     }
     EF_HIP(hipEventRecord(M->ev[st][0], M->stream));
 }
@@ -996,16 +998,19 @@ void setup_mixed(ef_mesh_s* M) {
 }
 
 // ----- sweeps ----------------------------------------------------------------
-// The upwards and the Dirichlet solve sweeps are captured once per (k, device pointers) into
-// a HIP graph and replayed with one hipGraphLaunch (EF_GRAPH=0 launches them one by one).
-// Captured work is kernels only: every allocation, descriptor upload and host check happens
-// before capture; graphs are dropped whenever the arenas or descriptor tables they point
-// into are reallocated.
+// The sweeps are launched kernel by kernel: queued launches follow each other on the device without a
+// gap, where a graph launch starts 6 us after the one before it has ended (two graphs a step: one
+// right-hand side on 64 leaves 60 us against 74 us, 64 on the adaptive Poisson mesh 1,674 against
+// 1,686 us).  EF_GRAPH=1 captures the upwards and the Dirichlet solve sweeps once per (k, device
+// pointers) into HIP graphs instead, replayed with one hipGraphLaunch each, for callers whose host
+// thread cannot spare the launches' 3 us each.  Captured work is kernels only: every allocation,
+// descriptor upload and host check happens before capture; graphs are dropped whenever the arenas or
+// descriptor tables they point into are reallocated.
 constexpr size_t MAX_GRAPHS = 64;
 
 bool graphs_on() {  // read on every sweep, so a process can compare both ways
     const char* e = std::getenv("EF_GRAPH");
-    return !(e && std::strcmp(e, "0") == 0) && !sync_check();
+    return e && std::strcmp(e, "0") != 0 && !sync_check();
 }
 
 void clear_graphs(ef_mesh_s* M) {
@@ -1114,6 +1119,24 @@ GemmLaunch tune_gemm(ef_mesh_s* M, const std::vector<TreeGemm>& probs, DevStore&
     return best;
 }
 
+// Split-K of a launch's products: k chunks per 16 x 16 tile so that the launch has about 1,024 waves
+// (one per SIMD) per 16 columns, and chunks of 128 for ranges of 512 and more; at most 16, of at least
+// 16 k values.  The rule counts row tiles and k ranges only, never the right-hand sides, so a column's
+// result is the same in any batch.  Launches of few tiles are as long as the dependent rounds of loads
+// over their k range: with the chunks of 128 alone one right-hand side took 77 us on 64 leaves and
+// 353 us on the adaptive Poisson mesh, so 60 and 333 us; twice the waves (2,048) gain 2 us more there
+// and lose 25 of 1,675 us at 64 right-hand sides, whose tiles fill the chip.
+void split_k(std::vector<TreeGemm>& probs) {
+    long long tiles = 0;
+    for (const TreeGemm& p : probs) tiles += (p.M + 15) / 16;
+    for (TreeGemm& p : probs) {
+        const int K = p.K0 + p.K1;
+        const long long fill = std::max<long long>(1024 / std::max<long long>(tiles, 1), K >= 512 ? K / 128 : 1);
+        const long long chunks = std::min<long long>({16, fill, K / 16});
+        p.kc = chunks < 2 ? 0 : (int)(((K + chunks - 1) / chunks + 15) / 16 * 16);
+    }
+}
+
 SweepPlan& sweep_plan(ef_mesh_s* M, int k) {
     auto it = M->sweeps.find(k);
     if (it != M->sweeps.end()) return *it->second;
@@ -1128,13 +1151,6 @@ SweepPlan& sweep_plan(ef_mesh_s* M, int k) {
     };
     const int D = P.maxdepth + 1;
     const int tn = k <= 16 ? 1 : 2;
-    // split-K for the long products of the upper levels (few merges, large operators): chunks
-    // of 128 once the concatenated k range reaches 512; the choice depends on the operator only,
-    // never on k, so a column's result is the same in any batch
-    auto split_kc = [](int K0, int K1) {
-        if (K0 + K1 < 512 || K0 % 128 != 0 || (K1 > 0 && K1 % 128 != 0)) return 0;
-        return 128;
-    };
     sp->lv.resize(D);
     for (int dd = 0; dd < D; dd++) {
         LevelSweep& L = sp->lv[dd];
@@ -1182,7 +1198,6 @@ SweepPlan& sweep_plan(ef_mesh_s* M, int k) {
             }
             p.D = V + nd.w_off; p.ldd = 1; p.dcs = (int)vrows;
             p.M = 4 * n; p.N = k;
-            p.kc = split_kc(p.K0, 0);
             pw.push_back(p);
             // h(q) += T_c(side q, interface sides) w(interfaces of c)   (mergeH_, the H block of child c)
             for (int q = 0; q < 8; q++) {
@@ -1200,7 +1215,6 @@ SweepPlan& sweep_plan(ef_mesh_s* M, int k) {
                 h.C = plain ? V + u.ch_off[c] + (long long)sq * n : h.D;
                 h.ldc = 1; h.ccs = (int)vrows; h.beta = 1.0;
                 h.M = n; h.N = k;
-                h.kc = split_kc(h.K0, h.K1);
                 ph.push_back(h);
             }
             // downward: u_int = S g + w   (applyS_, HPSAlgorithm.hpp:1194-1230), g read side by
@@ -1250,7 +1264,6 @@ SweepPlan& sweep_plan(ef_mesh_s* M, int k) {
             pd.D = V + nd.ui_off; pd.ldd = 1; pd.dcs = (int)vrows;
             if (!M->homogeneous_rhs) { pd.C = V + nd.w_off; pd.ldc = 1; pd.ccs = (int)vrows; pd.beta = 1.0; }
             pd.M = 4 * n; pd.N = k;
-            pd.kc = split_kc(pd.K0, 0);
             pu.push_back(pd);
             // uncoarsen_ steps: coarse gc -> ... -> g, alternating through gt
             for (int stp = 1; stp <= nd.tag; stp++) {
@@ -1273,6 +1286,9 @@ SweepPlan& sweep_plan(ef_mesh_s* M, int k) {
         L.interp_cnt = (int)ip.size();
         L.up_cnt = (int)ud.size();
         check_range(V, (size_t)vrows * k * 8, "vector arena");
+        split_k(pw);
+        split_k(ph);
+        split_k(pu);
         L.up = sp->store.stage(ud);
         L.copies = sp->store.stage(cp);
         L.interps = sp->store.stage(ip);
@@ -1484,7 +1500,9 @@ void do_solve_once(ef_mesh_s* M, const double* f_dev, const double* r_dev, const
             p.B0 = M->rootrhs.p; p.ldb0 = 1; p.bcs = m;
             p.D = V + root.g_off; p.ldd = 1; p.dcs = (int)P.vec_rows;
             p.M = m; p.N = k;
-            M->root_gemm = plan_gemm(std::vector<TreeGemm>{p}, k <= 16 ? 1 : 2, M->root_store, s);
+            std::vector<TreeGemm> pr{p};
+            split_k(pr);
+            M->root_gemm = plan_gemm(pr, k <= 16 ? 1 : 2, M->root_store, s);
             M->root_store.flush(s);
             M->root_sig = rsig;
         }

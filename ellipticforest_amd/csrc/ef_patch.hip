@@ -319,8 +319,9 @@ bool patch_constant(const double* c, long long NN) {
 
 void record_begin(ef_patches_s* p) {
     if (!p->ev[0]) {
-        EF_HIP(hipEventCreate(&p->ev[0]));
-        EF_HIP(hipEventCreate(&p->ev[1]));
+        // timing only: without a default event's system-scope release (2 us a record instead of 4)
+        EF_HIP(hipEventCreateWithFlags(&p->ev[0], hipEventDisableSystemFence));
+        EF_HIP(hipEventCreateWithFlags(&p->ev[1], hipEventDisableSystemFence));
     }
     EF_HIP(hipEventRecord(p->ev[0], p->stream));
 }

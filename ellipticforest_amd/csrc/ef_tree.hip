@@ -79,7 +79,7 @@ struct DiffRows {
     long long d2[4], d1[4];
 };
 
-template <int RT, int TN, bool F32, int MODE>
+template <int RT, int TN, bool F32, int MODE, int PD>
 __device__ inline void gemm_segment(const double* __restrict__ a0p, const double* __restrict__ a1p,
                                     const double* const (&bp)[TN], long long ldb, int K, double alpha,
                                     GemmAcc<F32> (&acc)[2][TN], const DiffRows& dr) {
@@ -160,11 +160,11 @@ __device__ inline void gemm_segment(const double* __restrict__ a0p, const double
         // blocks b + 1 .. b + PD - 1 are in flight, and block b + PD is issued into the slot b
         // frees -- no buffer is copied to another (a copy waits for its loads).  Measured at 64
         // right-hand sides, adaptive Poisson sweep GEMMs: PD = 2 0.871 ms, 3 0.969 ms, 4 0.996 ms
-        // (more registers, fewer waves per SIMD); a cur/next pair with a copy 0.948 ms.
+        // (more registers, fewer waves per SIMD); a cur/next pair with a copy 0.948 ms.  The split-K
+        // kernel, whose waves are few and whose ranges are short, takes PD = 3.
         // The steady-state loop issues its loads unconditionally, so the loop head sees one
         // order of outstanding loads and waits for the older block only (a conditional load
         // there makes the wait counts cover both blocks).
-        constexpr int PD = 2;
         Blk buf[PD];
         if (nfull >= PD) {
 #pragma unroll
@@ -188,8 +188,12 @@ __device__ inline void gemm_segment(const double* __restrict__ a0p, const double
             for (int j = 0; j < PD - 1; j++)
                 if (i + j < nfull) mma(buf[j]);
         } else {
-            load(0, buf[0]);
-            mma(buf[0]);
+#pragma unroll
+            for (int j = 0; j < PD - 1; j++)
+                if (j < nfull) load(16 * j, buf[j]);
+#pragma unroll
+            for (int j = 0; j < PD - 1; j++)
+                if (j < nfull) mma(buf[j]);
         }
         kb = 16 * nfull;
     }
@@ -282,15 +286,15 @@ tree_gemm_kernel(const TreeGemm* __restrict__ probs,
             for (int j = 0; j < TN; j++) bp[j] = p.B0 + (long long)cj[j] * p.bcs;
             const double* a0 = p.A0 + (long long)rows[0] * p.lda0 + kb0;
             const double* a1 = p.A0 + (long long)rows[RT - 1] * p.lda0 + kb0;
-            if (p.dsub) gemm_segment<RT, TN, F32, 1>(a0, a1, bp, 1, ke0 - kb0, p.alpha0, acc, dr);
-            else gemm_segment<RT, TN, F32, 2>(a0, a1, bp, 1, ke0 - kb0, p.alpha0, acc, dr);
+            if (p.dsub) gemm_segment<RT, TN, F32, 1, 2>(a0, a1, bp, 1, ke0 - kb0, p.alpha0, acc, dr);
+            else gemm_segment<RT, TN, F32, 2, 2>(a0, a1, bp, 1, ke0 - kb0, p.alpha0, acc, dr);
         } else {
 #pragma unroll
             for (int j = 0; j < TN; j++) bp[j] = p.B0 + (long long)kb0 * p.ldb0 + (long long)cj[j] * p.bcs;
             const double* a0 = p.A0 + (long long)rows[0] * p.lda0 + kb0;
             const double* a1 = p.A0 + (long long)rows[RT - 1] * p.lda0 + kb0;
-            if (p.ldb0 == 1) gemm_segment<RT, TN, F32, 0>(a0, a1, bp, 1, ke0 - kb0, p.alpha0, acc, dr);
-            else gemm_segment<RT, TN, F32, 3>(a0, a1, bp, p.ldb0, ke0 - kb0, p.alpha0, acc, dr);
+            if (p.ldb0 == 1) gemm_segment<RT, TN, F32, 0, 2>(a0, a1, bp, 1, ke0 - kb0, p.alpha0, acc, dr);
+            else gemm_segment<RT, TN, F32, 3, 2>(a0, a1, bp, p.ldb0, ke0 - kb0, p.alpha0, acc, dr);
         }
     }
     if (ke1 > kb1) {
@@ -299,8 +303,8 @@ tree_gemm_kernel(const TreeGemm* __restrict__ probs,
         for (int j = 0; j < TN; j++) bp[j] = p.B1 + (long long)kb1 * p.ldb1 + (long long)cj[j] * p.bcs;
         const double* a0 = p.A1 + (long long)rows[0] * p.lda1 + kb1;
         const double* a1 = p.A1 + (long long)rows[RT - 1] * p.lda1 + kb1;
-        if (p.ldb1 == 1) gemm_segment<RT, TN, F32, 0>(a0, a1, bp, 1, ke1 - kb1, p.alpha1, acc, dr);
-        else gemm_segment<RT, TN, F32, 3>(a0, a1, bp, p.ldb1, ke1 - kb1, p.alpha1, acc, dr);
+        if (p.ldb1 == 1) gemm_segment<RT, TN, F32, 0, 2>(a0, a1, bp, 1, ke1 - kb1, p.alpha1, acc, dr);
+        else gemm_segment<RT, TN, F32, 3, 2>(a0, a1, bp, p.ldb1, ke1 - kb1, p.alpha1, acc, dr);
     }
     // with RT = 1 both accumulator rows hold the same 16 rows; only the first is stored
 #pragma unroll
@@ -371,19 +375,19 @@ __global__ void __launch_bounds__(1024) tree_gemm_split_kernel(const TreeGemm* _
             const double* a0 = p.A0 + (long long)rowc * p.lda0 + kb0;
             if (p.dn > 0) {
                 bp[0] = p.B0 + (long long)cj * p.bcs;
-                if (p.dsub) gemm_segment<1, 1, false, 1>(a0, a0, bp, 1, ke0 - kb0, p.alpha0, acc, dr);
-                else gemm_segment<1, 1, false, 2>(a0, a0, bp, 1, ke0 - kb0, p.alpha0, acc, dr);
+                if (p.dsub) gemm_segment<1, 1, false, 1, 3>(a0, a0, bp, 1, ke0 - kb0, p.alpha0, acc, dr);
+                else gemm_segment<1, 1, false, 2, 3>(a0, a0, bp, 1, ke0 - kb0, p.alpha0, acc, dr);
             } else {
                 bp[0] = p.B0 + (long long)kb0 * p.ldb0 + (long long)cj * p.bcs;
-                if (p.ldb0 == 1) gemm_segment<1, 1, false, 0>(a0, a0, bp, 1, ke0 - kb0, p.alpha0, acc, dr);
-                else gemm_segment<1, 1, false, 3>(a0, a0, bp, p.ldb0, ke0 - kb0, p.alpha0, acc, dr);
+                if (p.ldb0 == 1) gemm_segment<1, 1, false, 0, 3>(a0, a0, bp, 1, ke0 - kb0, p.alpha0, acc, dr);
+                else gemm_segment<1, 1, false, 3, 3>(a0, a0, bp, p.ldb0, ke0 - kb0, p.alpha0, acc, dr);
             }
         }
         if (ke1 > kb1) {
             const double* bp[1] = {p.B1 + (long long)kb1 * p.ldb1 + (long long)cj * p.bcs};
             const double* a1 = p.A1 + (long long)rowc * p.lda1 + kb1;
-            if (p.ldb1 == 1) gemm_segment<1, 1, false, 0>(a1, a1, bp, 1, ke1 - kb1, p.alpha1, acc, dr);
-            else gemm_segment<1, 1, false, 3>(a1, a1, bp, p.ldb1, ke1 - kb1, p.alpha1, acc, dr);
+            if (p.ldb1 == 1) gemm_segment<1, 1, false, 0, 3>(a1, a1, bp, 1, ke1 - kb1, p.alpha1, acc, dr);
+            else gemm_segment<1, 1, false, 3, 3>(a1, a1, bp, p.ldb1, ke1 - kb1, p.alpha1, acc, dr);
         }
     }
     if (wave > 0) {

@@ -18,8 +18,8 @@
   works (up to ``nslots`` batches in flight); a batch completes when its event has fired.
   Requests that arrive while others are on the GPU join the next batch.
 * With ``buckets`` the batch width is rounded up to the next bucket (padding columns are
-  zero loads), so the sweep replays one of a few captured graphs; without it the width is
-  exact and the stages are launched one by one.
+  zero loads), so the sweep runs one of a few plans made when the mesh was admitted (and, with
+  EF_GRAPH=1, replays one of a few captured graphs); without it the width is exact.
 * Every right-hand side is reduced in an order that does not depend on the batch width, so
   a request's result is the same alone and in a batch.
 * Results stay in the slot's device buffer; a request that wants its solution on the host
