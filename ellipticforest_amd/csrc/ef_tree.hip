@@ -261,18 +261,20 @@ tree_gemm_kernel(const TreeGemm* __restrict__ probs,
     // C (when the product adds to it) loaded before the products, so its latency overlaps
     // them; rows and columns clamped as the stores are guarded
     double cv[RT][TN][4];
+    bool keep[TN];  // (a value that is not kept is dropped after the products: no wait before them)
     const bool has_c = p.C != nullptr;
     if (has_c) {
 #pragma unroll
-        for (int i = 0; i < RT; i++)
+        for (int j = 0; j < TN; j++) {
+            const int cb = p.cn > 0 ? cj[j] / p.cn : 0;
+            const double* cp = p.cn > 0 ? (cb == p.cb1 ? p.C1 : p.C) + (cj[j] - cb * p.cn) : p.C + (long long)cj[j] * p.ccs;
+            keep[j] = p.cn == 0 || cb == p.cb0 || cb == p.cb1;
 #pragma unroll
-            for (int j = 0; j < TN; j++)
+            for (int i = 0; i < RT; i++)
 #pragma unroll
-                for (int v = 0; v < 4; v++) {
-                    const int row = min(row0 + 16 * i + (F32 ? 4 * q + v : 4 * v + q), p.M - 1);
-                    const int col = min(col0 + 16 * j + r, p.N - 1);
-                    cv[i][j][v] = gld(p.C + (long long)row * p.ldc + (long long)col * p.ccs);
-                }
+                for (int v = 0; v < 4; v++)
+                    cv[i][j][v] = gld(cp + (long long)min(row0 + 16 * i + (F32 ? 4 * q + v : 4 * v + q), p.M - 1) * p.ldc);
+        }
     }
     DiffRows dr;
     dr.dn = p.dn;
@@ -316,7 +318,7 @@ tree_gemm_kernel(const TreeGemm* __restrict__ probs,
                 const int row = row0 + 16 * i + (F32 ? 4 * q + v : 4 * v + q), col = col0 + 16 * j + r;
                 if (row < p.M && col < p.N) {
                     double o = (double)acc[i][j][v];
-                    if (has_c) o += p.beta * cv[i][j][v];
+                    if (has_c) o += keep[j] ? p.beta * cv[i][j][v] : 0.0;
                     *gmem(p.D + (long long)row * p.ldd + (long long)col * p.dcs) = o;
                 }
             }
@@ -1419,31 +1421,22 @@ __global__ void __launch_bounds__(256) tree_assemble_kernel(const AsmDesc* __res
     const AsmDesc d = descs[blockIdx.y];
     const int n = d.n;
     const long long n2 = (long long)n * n;
-    long long e = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (e >= 80 * n2) return;
-    if (e < 16 * n2) {  // X (mergeX_, HPSAlgorithm.hpp:870-895), interface order [ag, bo, ab, go]
-        const int row = (int)(e / (4 * n)), col = (int)(e % (4 * n));
-        const int ri = row / n, i = row % n, ci = col / n, j = col % n;
-        const int c1 = if_c1(ri), s1 = if_s1(ri), c2 = if_c2(ri), s2 = if_s2(ri);
-        double v;
-        if (ri == ci) {
-            v = tblk(pick4(d.Tc, c1), n, s1, s1, i, j) - tblk(pick4(d.Tc, c2), n, s2, s2, i, j);
-        } else {
-            const int sc1 = side_on_if(c1, ci), sc2 = side_on_if(c2, ci);
-            v = 0.0;
-            if (sc1 >= 0) v = tblk(pick4(d.Tc, c1), n, s1, sc1, i, j);
-            else if (sc2 >= 0) v = -tblk(pick4(d.Tc, c2), n, s2, sc2, i, j);
-        }
-        d.X[e] = v;
-        return;
+    const long long e = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (e >= 16 * n2) return;
+    // X (mergeX_, HPSAlgorithm.hpp:870-895), interface order [ag, bo, ab, go]
+    const int row = (int)(e / (4 * n)), col = (int)(e % (4 * n));
+    const int ri = row / n, i = row % n, ci = col / n, j = col % n;
+    const int c1 = if_c1(ri), s1 = if_s1(ri), c2 = if_c2(ri), s2 = if_s2(ri);
+    double v;
+    if (ri == ci) {
+        v = tblk(pick4(d.Tc, c1), n, s1, s1, i, j) - tblk(pick4(d.Tc, c2), n, s2, s2, i, j);
+    } else {
+        const int sc1 = side_on_if(c1, ci), sc2 = side_on_if(c2, ci);
+        v = 0.0;
+        if (sc1 >= 0) v = tblk(pick4(d.Tc, c1), n, s1, sc1, i, j);
+        else if (sc2 >= 0) v = -tblk(pick4(d.Tc, c2), n, s2, sc2, i, j);
     }
-    e -= 16 * n2;
-    // T block diagonal (mergeT_ :940-968 before H S is added), WESN rows and columns
-    const int row = (int)(e / (8 * n)), col = (int)(e % (8 * n));
-    const int q = row / n, i = row % n, q2 = col / n, j = col % n;
-    double v = 0.0;
-    if (q_child(q) == q_child(q2)) v = tblk(pick4(d.Tc, q_child(q)), n, q_side(q), q_side(q2), i, j);
-    d.T[e] = v;
+    d.X[e] = v;
 }
 
 // L12 of fine size nf (SpecialMatrices.hpp:136-173), column b: rows 0 (b <= 2), 2b-1 and 2b
@@ -1652,7 +1645,11 @@ GemmLaunch plan_gemm(const std::vector<TreeGemm>& probs_in, int tn, DevStore& st
         if (p.M <= 0 || p.N <= 0) { p.kc = 0; continue; }
         // extents: the kernel clamps rows to M-1, columns to N-1 and k to K-1
         check_strided(p.D, p.M, p.N, p.ldd, p.dcs, "GEMM D");
-        if (p.C) check_strided(p.C, p.M, p.N, p.ldc, p.ccs, "GEMM C");
+        if (p.cn > 0) {
+            if (p.kc > 0 || !p.C || !p.C1) throw EfError(EF_ERR_INTERNAL, "GEMM with C in blocks needs both blocks and no split");
+            check_strided(p.C, p.M, p.cn, p.ldc, 1, "GEMM C block");
+            check_strided(p.C1, p.M, p.cn, p.ldc, 1, "GEMM C block");
+        } else if (p.C) check_strided(p.C, p.M, p.N, p.ldc, p.ccs, "GEMM C");
         const double* As[2] = {p.A0, p.A1};
         const double* Bs[2] = {p.B0, p.B1};
         const int lda[2] = {p.lda0, p.lda1}, ldb[2] = {p.ldb0, p.ldb1}, K[2] = {p.K0, p.K1};

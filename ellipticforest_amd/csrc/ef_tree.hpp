@@ -91,8 +91,12 @@ struct TreeGemm {
     // a node's g read where they lie.
     int dn, dsub;
     long long d2[4], d1[4];
+    // Block mode of C (cn > 0, ccs = 1): C is zero but for the column blocks cb0 and cb1 (of cn columns
+    // each), which are the cn columns at C and at C1: T = blkdiag + H S read from the child's DtN.
+    const double* C1;
+    int cn, cb0, cb1, pad2;
 };
-static_assert(sizeof(TreeGemm) == 208, "TreeGemm layout");
+static_assert(sizeof(TreeGemm) == 232, "TreeGemm layout");
 
 // F32: operands rounded to FP32, v_mfma_f32_16x16x4_f32 with FP32 accumulation, FP64 output
 // (+ beta C in FP64); the mixed-precision build's S and T products.
@@ -165,8 +169,7 @@ __global__ void inv_mult_kernel(const double* A, double* Mm, const double* Pn, i
 __global__ void inv_update_kernel(const double* Wa, double* Wb, const double* Mm, double* Pn, int m, int k, int* flag);
 
 // ---------------------------------------------------------------------------------------
-// Merge assembly (createMatrixBlocks_ + mergeX_ + the block-diagonal part of mergeT_,
-// HPSAlgorithm.hpp:799-968, with the WESN order of reorderOperators_, :979-993): from the
+// Merge assembly (createMatrixBlocks_ + mergeX_, HPSAlgorithm.hpp:799-895): from the
 // four children's DtN maps (each 4n x 4n, coarsened), X (4n x 4n) into the inversion work
 // buffer and T (8n x 8n, WESN rows and columns) = diag blocks T_c(tau side, tau side).
 // ---------------------------------------------------------------------------------------
