@@ -834,6 +834,9 @@ void check_tree_kernels() {
     check_kernel_resources((const void*)tree_gemm_kernel<2, 2, false>, "tree_gemm_kernel<2,2>");
     check_kernel_resources((const void*)tree_gemm_kernel<1, 2, false>, "tree_gemm_kernel<1,2>");
     check_kernel_resources((const void*)tree_gemm_kernel<1, 2, true>, "tree_gemm_kernel<1,2,f32>");
+    check_kernel_resources((const void*)tree_gemm_lds_kernel<1, 4>, "tree_gemm_lds_kernel<1,4>");
+    check_kernel_resources((const void*)tree_gemm_lds_kernel<2, 2>, "tree_gemm_lds_kernel<2,2>");
+    check_kernel_resources((const void*)tree_gemm_lds_kernel<4, 1>, "tree_gemm_lds_kernel<4,1>");
     check_kernel_resources((const void*)tree_gemm_kernel<1, 1, true>, "tree_gemm_kernel<1,1,f32>");
     check_kernel_resources((const void*)tree_gemm_kernel<2, 2, true>, "tree_gemm_kernel<2,2,f32>");
     check_kernel_resources((const void*)tree_gemm_split_kernel, "tree_gemm_split_kernel");

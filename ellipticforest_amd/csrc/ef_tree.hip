@@ -65,7 +65,7 @@ __device__ inline double readlane_f64(double x, int src) {
 // ---------------------------------------------------------------------------------------
 // Batched GEMM
 // ---------------------------------------------------------------------------------------
-// alpha * A B over k in [0, K) into this wave's 32 x (16 TN) block.  a0p / a1p: the lane's two
+// A B over k in [0, K) into this wave's 32 x (16 TN) block.  a0p / a1p: the lane's two
 // A rows (r and r + 16, clamped into the matrix); bp[j]: B column (clamped) of column tile j.
 // Within each block of 16 k values lane group q takes k = kb + 4q + s at MFMA step s: A is
 // read as two 16-byte vectors per lane and row (a 128-byte row segment per lane group), B as
@@ -79,9 +79,19 @@ struct DiffRows {
     long long d2[4], d1[4];
 };
 
+// The factors alpha of a product's two segments are signs, applied to the accumulators once per segment
+// (A scaled as it is loaded took a multiplication per MFMA on the unit the f64 MFMAs run on).
+template <bool F32, int TN>
+__device__ inline void flip_sign(GemmAcc<F32> (&acc)[2][TN]) {
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) acc[i][j] = -acc[i][j];
+}
+
 template <int RT, int TN, bool F32, int MODE, int PD>
 __device__ inline void gemm_segment(const double* __restrict__ a0p, const double* __restrict__ a1p,
-                                    const double* const (&bp)[TN], long long ldb, int K, double alpha,
+                                    const double* const (&bp)[TN], long long ldb, int K,
                                     GemmAcc<F32> (&acc)[2][TN], const DiffRows& dr) {
     constexpr bool DIFF = MODE == 1 || MODE == 2;
     const int q = (int)(threadIdx.x & 63) >> 4;
@@ -139,10 +149,10 @@ __device__ inline void gemm_segment(const double* __restrict__ a0p, const double
         }
     };
     auto mma = [&](const Blk& o) {
-        const double a0[4] = {alpha * o.x0[0], alpha * o.x0[1], alpha * o.x1[0], alpha * o.x1[1]};
+        const double a0[4] = {o.x0[0], o.x0[1], o.x1[0], o.x1[1]};
         double a1[4] = {0.0, 0.0, 0.0, 0.0};
         if (RT == 2) {
-            a1[0] = alpha * o.y0[0]; a1[1] = alpha * o.y0[1]; a1[2] = alpha * o.y1[0]; a1[3] = alpha * o.y1[1];
+            a1[0] = o.y0[0]; a1[1] = o.y0[1]; a1[2] = o.y1[0]; a1[3] = o.y1[1];
         }
 #pragma unroll
         for (int s = 0; s < 4; s++)
@@ -205,10 +215,10 @@ __device__ inline void gemm_segment(const double* __restrict__ a0p, const double
             const bool ok = k + s < K;
             const int kk = ok ? k + s : K - 1;
             const double x = gld(a0p + kk);
-            a0[s] = ok ? alpha * x : 0.0;
+            a0[s] = ok ? x : 0.0;
             if (RT == 2) {
                 const double y = gld(a1p + kk);
-                a1[s] = ok ? alpha * y : 0.0;
+                a1[s] = ok ? y : 0.0;
             }
             if (DIFF) {
                 long long o2, o1;
@@ -288,27 +298,29 @@ tree_gemm_kernel(const TreeGemm* __restrict__ probs,
             for (int j = 0; j < TN; j++) bp[j] = p.B0 + (long long)cj[j] * p.bcs;
             const double* a0 = p.A0 + (long long)rows[0] * p.lda0 + kb0;
             const double* a1 = p.A0 + (long long)rows[RT - 1] * p.lda0 + kb0;
-            if (p.dsub) gemm_segment<RT, TN, F32, 1, 2>(a0, a1, bp, 1, ke0 - kb0, p.alpha0, acc, dr);
-            else gemm_segment<RT, TN, F32, 2, 2>(a0, a1, bp, 1, ke0 - kb0, p.alpha0, acc, dr);
+            if (p.dsub) gemm_segment<RT, TN, F32, 1, 2>(a0, a1, bp, 1, ke0 - kb0, acc, dr);
+            else gemm_segment<RT, TN, F32, 2, 2>(a0, a1, bp, 1, ke0 - kb0, acc, dr);
         } else {
 #pragma unroll
             for (int j = 0; j < TN; j++) bp[j] = p.B0 + (long long)kb0 * p.ldb0 + (long long)cj[j] * p.bcs;
             const double* a0 = p.A0 + (long long)rows[0] * p.lda0 + kb0;
             const double* a1 = p.A0 + (long long)rows[RT - 1] * p.lda0 + kb0;
-            if (p.ldb0 == 1) gemm_segment<RT, TN, F32, 0, 2>(a0, a1, bp, 1, ke0 - kb0, p.alpha0, acc, dr);
-            else gemm_segment<RT, TN, F32, 3, 2>(a0, a1, bp, p.ldb0, ke0 - kb0, p.alpha0, acc, dr);
+            if (p.ldb0 == 1) gemm_segment<RT, TN, F32, 0, 2>(a0, a1, bp, 1, ke0 - kb0, acc, dr);
+            else gemm_segment<RT, TN, F32, 3, 2>(a0, a1, bp, p.ldb0, ke0 - kb0, acc, dr);
         }
     }
     if (ke1 > kb1) {
+        if (p.alpha0 != p.alpha1) flip_sign<F32>(acc);
         const double* bp[TN];
 #pragma unroll
         for (int j = 0; j < TN; j++) bp[j] = p.B1 + (long long)kb1 * p.ldb1 + (long long)cj[j] * p.bcs;
         const double* a0 = p.A1 + (long long)rows[0] * p.lda1 + kb1;
         const double* a1 = p.A1 + (long long)rows[RT - 1] * p.lda1 + kb1;
-        if (p.ldb1 == 1) gemm_segment<RT, TN, F32, 0, 2>(a0, a1, bp, 1, ke1 - kb1, p.alpha1, acc, dr);
-        else gemm_segment<RT, TN, F32, 3, 2>(a0, a1, bp, p.ldb1, ke1 - kb1, p.alpha1, acc, dr);
+        if (p.ldb1 == 1) gemm_segment<RT, TN, F32, 0, 2>(a0, a1, bp, 1, ke1 - kb1, acc, dr);
+        else gemm_segment<RT, TN, F32, 3, 2>(a0, a1, bp, p.ldb1, ke1 - kb1, acc, dr);
     }
-    // with RT = 1 both accumulator rows hold the same 16 rows; only the first is stored
+    if ((ke1 > kb1 ? p.alpha1 : p.alpha0) < 0.0) flip_sign<F32>(acc);
+    // with RT = 1 only the first accumulator row holds products
 #pragma unroll
     for (int i = 0; i < RT; i++)
 #pragma unroll
@@ -330,6 +342,140 @@ template __global__ void tree_gemm_kernel<2, 2, false>(const TreeGemm*, const in
 template __global__ void tree_gemm_kernel<1, 1, true>(const TreeGemm*, const int*, const int*, int);
 template __global__ void tree_gemm_kernel<1, 2, true>(const TreeGemm*, const int*, const int*, int);
 template __global__ void tree_gemm_kernel<2, 2, true>(const TreeGemm*, const int*, const int*, int);
+
+// The build's S and T products of merges with n >= 32 (row-major operands, K a multiple of 16, M and N of
+// the tile): one workgroup per (32 WR) x (32 WC) tile of D, its WR x WC waves a 32 x 32 block each, A and
+// B staged through LDS in blocks of 16 k values, two blocks' loads in flight during the MFMAs of the
+// one before.  Bound: the f64 matrix cores.  One wave per 32 x 32 block reading its own operands
+// (tree_gemm_kernel) asks the L1 for 32 bytes per cycle and CU at full matrix rate and holds 2 waves per
+// SIMD; LDS tiles halve that and 4 waves fit.  n = 512, T (34 GFLOP): 724 us (47 TFLOP/s) -> 554
+// (62; the card's large matrix product reaches 72); 256 merges of n = 32: S 48 -> 42, T 97 -> 78 us; S and
+// T of 1,024 leaves of 32^2: 2.32 -> 1.79 ms.  Of that: one block in flight instead of two 604 us
+// for the n = 512 product; workgroups in launch order, so that each XCD's L2 sees every tile, 578.
+// Each element sums its k range in tree_gemm_kernel's order, so the two agree in every bit.
+template <int WR, int WC>
+__global__ void __launch_bounds__(256) tree_gemm_lds_kernel(const TreeGemm* __restrict__ probs,
+                                                            const int* __restrict__ start,
+                                                            const int* __restrict__ gprob, int ngroups) {
+    static_assert(WR * WC == 4, "four waves");
+    constexpr int TR = 32 * WR, TC = 32 * WC;
+    constexpr int LA = 18, LB = TC + 4;  // LDS rows of A and B in doubles: each read covers every bank once
+    __shared__ __attribute__((aligned(16))) double sa[2][TR * LA];
+    __shared__ __attribute__((aligned(16))) double sb[2][16 * LB];
+    const int bid = (int)blockIdx.x, n8 = ngroups / 8;
+    if (bid >= ngroups) return;  // uniform per workgroup
+    // (consecutive workgroups go to the 8 XCDs in turn: each gets a run of consecutive tiles)
+    const int g = bid < 8 * n8 ? (bid & 7) * n8 + (bid >> 3) : bid;
+    const int lo = __builtin_amdgcn_readfirstlane(gprob[g]);
+    const TreeGemm p = probs[lo];
+    const int tid = threadIdx.x, lane = tid & 63, q = lane >> 4, r = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int t = g - start[lo], tm = p.M / TR;
+    const int row0 = (t % tm) * TR, col0 = (t / tm) * TC;
+    const int wr = 32 * (wave / WC), wc = 32 * (wave % WC);
+    GemmAcc<false> acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) acc[i][j] = GemmAcc<false>{0, 0, 0, 0};
+    const int nb0 = p.K0 / 16, nb = nb0 + p.K1 / 16;
+    struct Blk {
+        td2 x[WR], y[WC];
+    };
+    // a lane's share of a block: WR vectors of A (eight to a row), WC of B (16 WC to a row)
+    auto load = [&](int b, Blk& o) {  // block b of the concatenated k range (past its end: the last one again)
+        b = min(b, nb - 1);
+        const bool s1 = b >= nb0;  // uniform
+        const int k = 16 * (s1 ? b - nb0 : b);
+        const double* A = (s1 ? p.A1 : p.A0) + k;
+        const double* B = (s1 ? p.B1 : p.B0) + col0;
+        const int lda = s1 ? p.lda1 : p.lda0, ldb = s1 ? p.ldb1 : p.ldb0;
+#pragma unroll
+        for (int v = 0; v < WR; v++) o.x[v] = gld2(A + (long long)(row0 + 32 * v + (tid >> 3)) * lda + 2 * (tid & 7));
+#pragma unroll
+        for (int v = 0; v < WC; v++) {
+            const int e = tid + 256 * v;
+            o.y[v] = gld2(B + (long long)(k + e / (16 * WC)) * ldb + 2 * (e % (16 * WC)));
+        }
+    };
+    auto stage = [&](int slot, const Blk& o) {
+#pragma unroll
+        for (int v = 0; v < WR; v++) *(td2*)&sa[slot][(32 * v + (tid >> 3)) * LA + 2 * (tid & 7)] = o.x[v];
+#pragma unroll
+        for (int v = 0; v < WC; v++) {
+            const int e = tid + 256 * v;
+            *(td2*)&sb[slot][e / (16 * WC) * LB + 2 * (e % (16 * WC))] = o.y[v];
+        }
+    };
+    Blk buf[2];
+    load(0, buf[0]);
+    load(1, buf[1]);
+    stage(0, buf[0]);
+    __syncthreads();
+    for (int b0 = 0; b0 < nb; b0 += 2) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int b = b0 + h;
+            if (b >= nb) break;  // uniform
+            if (b == nb0 && p.alpha0 != p.alpha1) flip_sign<false>(acc);
+            load(b + 2, buf[h]);
+            const double* la = &sa[h][(wr + r) * LA + 4 * q];
+            const double* lb = &sb[h][4 * q * LB + wc + r];
+            double a[2][4], v[2][4];
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                const td2 u0 = *(const td2*)(la + 16 * i * LA), u1 = *(const td2*)(la + 16 * i * LA + 2);
+                a[i][0] = u0[0]; a[i][1] = u0[1]; a[i][2] = u1[0]; a[i][3] = u1[1];
+            }
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int s = 0; s < 4; s++) v[j][s] = lb[s * LB + 16 * j];
+#pragma unroll
+            for (int s = 0; s < 4; s++)
+#pragma unroll
+                for (int j = 0; j < 2; j++)
+#pragma unroll
+                    for (int i = 0; i < 2; i++) acc[i][j] = mfma_f64(a[i][s], v[j][s], acc[i][j]);
+            stage(1 - h, buf[1 - h]);  // (block b - 1 was read from that slot: every wave is past the barrier after it)
+            __syncthreads();
+        }
+    }
+    if ((p.K1 > 0 ? p.alpha1 : p.alpha0) < 0.0) flip_sign<false>(acc);
+    // C: a wave's columns lie in one column block (cn a multiple of 32)
+    const int cb = p.cn > 0 ? (col0 + wc) / p.cn : 0;
+    const double* C = p.C;
+    if (p.cn > 0) C = cb == p.cb0 ? p.C - (long long)cb * p.cn : cb == p.cb1 ? p.C1 - (long long)cb * p.cn : nullptr;
+    if (C) {  // uniform
+        double cv[2][2][4];
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int v = 0; v < 4; v++)
+                    cv[i][j][v] = gld(C + (long long)(row0 + wr + 16 * i + 4 * v + q) * p.ldc + col0 + wc + 16 * j + r);
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int v = 0; v < 4; v++) acc[i][j][v] += p.beta * cv[i][j][v];
+    }
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int row = row0 + wr + 16 * i + 4 * v + q, col = col0 + wc + 16 * j + r;
+                *gmem(p.D + (long long)row * p.ldd + col) = acc[i][j][v];
+            }
+}
+
+template __global__ void tree_gemm_lds_kernel<1, 4>(const TreeGemm*, const int*, const int*, int);
+template __global__ void tree_gemm_lds_kernel<2, 2>(const TreeGemm*, const int*, const int*, int);
+template __global__ void tree_gemm_lds_kernel<4, 1>(const TreeGemm*, const int*, const int*, int);
 
 // Split-K inside the workgroup: workgroup g computes the 16 x 16 output tile g - start[p] of
 // problem p = gprob[g]; its wave w sums chunk w, k in [w kc, (w + 1) kc), of the concatenated k
@@ -377,20 +523,22 @@ __global__ void __launch_bounds__(1024) tree_gemm_split_kernel(const TreeGemm* _
             const double* a0 = p.A0 + (long long)rowc * p.lda0 + kb0;
             if (p.dn > 0) {
                 bp[0] = p.B0 + (long long)cj * p.bcs;
-                if (p.dsub) gemm_segment<1, 1, false, 1, 3>(a0, a0, bp, 1, ke0 - kb0, p.alpha0, acc, dr);
-                else gemm_segment<1, 1, false, 2, 3>(a0, a0, bp, 1, ke0 - kb0, p.alpha0, acc, dr);
+                if (p.dsub) gemm_segment<1, 1, false, 1, 3>(a0, a0, bp, 1, ke0 - kb0, acc, dr);
+                else gemm_segment<1, 1, false, 2, 3>(a0, a0, bp, 1, ke0 - kb0, acc, dr);
             } else {
                 bp[0] = p.B0 + (long long)kb0 * p.ldb0 + (long long)cj * p.bcs;
-                if (p.ldb0 == 1) gemm_segment<1, 1, false, 0, 3>(a0, a0, bp, 1, ke0 - kb0, p.alpha0, acc, dr);
-                else gemm_segment<1, 1, false, 3, 3>(a0, a0, bp, p.ldb0, ke0 - kb0, p.alpha0, acc, dr);
+                if (p.ldb0 == 1) gemm_segment<1, 1, false, 0, 3>(a0, a0, bp, 1, ke0 - kb0, acc, dr);
+                else gemm_segment<1, 1, false, 3, 3>(a0, a0, bp, p.ldb0, ke0 - kb0, acc, dr);
             }
         }
         if (ke1 > kb1) {
+            if (p.alpha0 != p.alpha1) flip_sign<false>(acc);
             const double* bp[1] = {p.B1 + (long long)kb1 * p.ldb1 + (long long)cj * p.bcs};
             const double* a1 = p.A1 + (long long)rowc * p.lda1 + kb1;
-            if (p.ldb1 == 1) gemm_segment<1, 1, false, 0, 3>(a1, a1, bp, 1, ke1 - kb1, p.alpha1, acc, dr);
-            else gemm_segment<1, 1, false, 3, 3>(a1, a1, bp, p.ldb1, ke1 - kb1, p.alpha1, acc, dr);
+            if (p.ldb1 == 1) gemm_segment<1, 1, false, 0, 3>(a1, a1, bp, 1, ke1 - kb1, acc, dr);
+            else gemm_segment<1, 1, false, 3, 3>(a1, a1, bp, p.ldb1, ke1 - kb1, acc, dr);
         }
+        if ((ke1 > kb1 ? p.alpha1 : p.alpha0) < 0.0) flip_sign<false>(acc);
     }
     if (wave > 0) {
 #pragma unroll
@@ -1602,6 +1750,17 @@ __global__ void __launch_bounds__(256) tree_root_robin_kernel(const double* T, c
 // ---------------------------------------------------------------------------------------
 // Host side
 // ---------------------------------------------------------------------------------------
+// tree_gemm_lds_kernel's products on tr x tc tiles: whole tiles and blocks of k only, so no load is clamped.
+// It is the faster one from its smallest launch (64 workgroups, n = 64: S 11.3 -> 10.9 us, T 12.5 -> 11.2) on; the
+// square tile is taken where it fits (a third less operand traffic than 32 x 128).
+static bool fits_lds_tiles(const TreeGemm& p, int tr, int tc) {
+    auto row_major = [](int cs) { return cs == 0 || cs == 1; };
+    auto vectors = [](const double* b, int ld) { return ((uintptr_t)b & 15) == 0 && (ld & 1) == 0; };
+    return p.M > 0 && p.N > 0 && p.M % tr == 0 && p.N % tc == 0 && p.dn == 0 && p.K0 > 0 && p.K0 % 16 == 0 &&
+           p.K1 % 16 == 0 && row_major(p.bcs) && row_major(p.ccs) && row_major(p.dcs) && p.cn % 32 == 0 && p.ldb0 > 1 &&
+           vectors(p.B0, p.ldb0) && (p.K1 == 0 || (p.ldb1 > 1 && vectors(p.B1, p.ldb1)));
+}
+
 GemmLaunch plan_gemm(const std::vector<TreeGemm>& probs_in, int tn, DevStore& store, hipStream_t s, bool f32, int rt) {
     GemmLaunch g;
     g.tn = tn;
@@ -1632,8 +1791,14 @@ GemmLaunch plan_gemm(const std::vector<TreeGemm>& probs_in, int tn, DevStore& st
         g.kw = kw;
         g.rt = g.tn = 1;
     }
+    if (kw == 1 && !f32 && tn == 2 && rt == 0)
+        for (int wr : {2, 1, 4}) {
+            bool fit = g.lds == 0;
+            for (const TreeGemm& p : probs) fit = fit && fits_lds_tiles(p, 32 * wr, 128 / wr);
+            if (fit) g.lds = wr;
+        }
     std::vector<int> start(probs.size() + 1, 0);
-    const int rw = 16 * g.rt, cw = 16 * g.tn;
+    const int rw = g.lds ? 32 * g.lds : 16 * g.rt, cw = g.lds ? 128 / g.lds : 16 * g.tn;
     long long total = 0;
     for (size_t i = 0; i < probs.size(); i++) {
         TreeGemm& p = probs[i];
@@ -1643,6 +1808,8 @@ GemmLaunch plan_gemm(const std::vector<TreeGemm>& probs_in, int tn, DevStore& st
         if (p.ccs == 0) p.ccs = 1;
         if (p.dcs == 0) p.dcs = 1;
         if (p.M <= 0 || p.N <= 0) { p.kc = 0; continue; }
+        if (std::abs(p.alpha0) != 1.0 || (p.K1 > 0 && std::abs(p.alpha1) != 1.0))
+            throw EfError(EF_ERR_INTERNAL, "GEMM segment factor other than 1 and -1");
         // extents: the kernel clamps rows to M-1, columns to N-1 and k to K-1
         check_strided(p.D, p.M, p.N, p.ldd, p.dcs, "GEMM D");
         if (p.cn > 0) {
@@ -1709,6 +1876,16 @@ void run_gemm(const GemmLaunch& g, hipStream_t s) {
                   g.start, g.wprob, g.nwaves);
         return;
     }
+#define EF_GEMM_LAUNCH(WR_, WC_, NAME_)                                                                       \
+    EF_LAUNCH(NAME_, (tree_gemm_lds_kernel<WR_, WC_>), dim3(g.nwaves), dim3(256), s, g.probs, g.start, g.wprob, \
+              g.nwaves)
+    if (g.lds > 0) {
+        if (g.lds == 1) EF_GEMM_LAUNCH(1, 4, "tree_gemm_lds_kernel<1,4>");
+        else if (g.lds == 2) EF_GEMM_LAUNCH(2, 2, "tree_gemm_lds_kernel<2,2>");
+        else EF_GEMM_LAUNCH(4, 1, "tree_gemm_lds_kernel<4,1>");
+        return;
+    }
+#undef EF_GEMM_LAUNCH
     const dim3 grid(blocks_for(g.nwaves, 4)), block(256);
 #define EF_GEMM_LAUNCH(RT_, TN_, F32_, NAME_)                                                          \
     EF_LAUNCH(NAME_, (tree_gemm_kernel<RT_, TN_, F32_>), grid, block, s, g.probs, g.start, g.wprob, g.nwaves)

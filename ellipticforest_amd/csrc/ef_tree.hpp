@@ -103,6 +103,8 @@ static_assert(sizeof(TreeGemm) == 232, "TreeGemm layout");
 template <int RT, int TN, bool F32>
 __global__ void tree_gemm_kernel(const TreeGemm* probs, const int* start, const int* wprob, int nwaves);
 __global__ void tree_gemm_split_kernel(const TreeGemm* probs, const int* start, const int* gprob, int ngroups);
+template <int WR, int WC>
+__global__ void tree_gemm_lds_kernel(const TreeGemm* probs, const int* start, const int* gprob, int ngroups);
 
 // ---------------------------------------------------------------------------------------
 // In-place blocked Gauss-Jordan inversion with partial pivoting of a batch of B equally
@@ -214,6 +216,7 @@ struct GemmLaunch {
     int nprob = 0, nwaves = 0, rt = 2, tn = 2;
     int kw = 0;                   // > 1: split-K launch, waves per 16 x 16 tile
     bool f32 = false;  // FP32 matrix cores (mixed precision)
+    int lds = 0;       // > 0: tree_gemm_lds_kernel<lds, 4 / lds> (wprob: problem of each workgroup)
 };
 // Checks every problem (extents inside their allocations, alignment), sets the split-K chunks of
 // a split launch, stages problems and wave offsets in `store` (device memory the caller keeps
