@@ -5,13 +5,14 @@
 //
 // The reference forms X, S_RHS and H element by element, calls dgesv for S = X^-1 S_RHS and
 // dgemm for T = blkdiag + H S (Matrix.hpp:827-953), one family at a time.  Here:
-//  * X is inverted once per merge (blocked Gauss-Jordan with partial pivoting, every O(m^3)
-//    step a batched MFMA product), so the upward sweep's mergeW_ is a product with X^-1
-//    instead of a re-factorisation per solve;
+//  * X is inverted once per merge (blocked Gauss-Jordan in natural order with the multipliers
+//    checked, redone with partial pivoting where one is large; every O(m^3) step a batched
+//    MFMA product), so the upward sweep's mergeW_ is a product with X^-1 instead of a
+//    re-factorisation per solve;
 //  * S = X^-1 S_RHS and T = blkdiag + H S read S_RHS and H straight out of the children's
 //    DtN maps (they are blocks of them, with signs), skipping their zero blocks;
-//  * every product runs on one register-resident batched GEMM kernel whose waves read their
-//    operands in the v_mfma_f64_16x16x4_f64 layouts (no LDS, no scratch).
+//  * the sweeps' products run on register-resident batched GEMM kernels whose waves read their
+//    operands in the v_mfma_f64_16x16x4_f64 layouts, the build's larger ones on tiles in LDS.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -352,7 +353,7 @@ template __global__ void tree_gemm_kernel<2, 2, true>(const TreeGemm*, const int
 // (62; the card's large matrix product reaches 72); 256 merges of n = 32: S 48 -> 42, T 97 -> 78 us; S and
 // T of 1,024 leaves of 32^2: 2.32 -> 1.79 ms.  Of that: one block in flight instead of two 604 us
 // for the n = 512 product; workgroups in launch order, so that each XCD's L2 sees every tile, 578.
-// Each element sums its k range in tree_gemm_kernel's order, so the two agree in every bit.
+// Each element sums its k range in the same order as there.
 template <int WR, int WC>
 __global__ void __launch_bounds__(256) tree_gemm_lds_kernel(const TreeGemm* __restrict__ probs,
                                                             const int* __restrict__ start,
