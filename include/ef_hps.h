@@ -198,8 +198,9 @@ int ef_mesh_eval_load(ef_mesh mesh, const double* params_dev, int nrhs, double* 
  * stream over whatever the vector arena holds; ms per pass and kernel launches per pass. */
 int ef_mesh_time_sweep_gemms(ef_mesh mesh, int nrhs, int reps, double* ms_per_pass, int* launches);
 
-/* Diagnostic: the batched inversion every merge uses (blocked Gauss-Jordan with partial
- * pivoting, tournament pivoting over 512-row chunks), applied to B host matrices of order m
+/* Diagnostic: the pivoted batched inversion (blocked Gauss-Jordan with partial pivoting,
+ * tournament pivoting over 512-row chunks) that the merges fall back to where an inversion in
+ * natural order meets a large multiplier, applied to B host matrices of order m
  * (row-major, B x m x m).  Ainv receives the inverses; ipiv (B x m, may be NULL) the
  * LAPACK-order row interchanges (0-based: position c was exchanged with ipiv[c]), equal to
  * dgetrf's wherever no step spans more than one chunk (m <= 512).  Replaces the LU of the
