@@ -8,10 +8,10 @@ Source transforms (applied to copies under tests/cpu_emu/_build/):
 """
 from __future__ import annotations
 
+import concurrent.futures
 import os
 import re
 import subprocess
-import sys
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(os.path.dirname(HERE))
@@ -58,12 +58,24 @@ def build():
         with open(dst, "w") as f:
             f.write(t)
     srcs = [os.path.join(OUT, n.replace(".hip", ".cpp")) for n in SOURCES] + [os.path.join(HERE, "hip_cpu_shim.cpp")]
-    cmd = [clangxx(), "-std=c++20", os.environ.get("EF_EMU_OPT", "-O1"), "-g"] + os.environ.get("EF_EMU_SAN", "").split() + [ "-fPIC", "-shared", "-pthread", "-I", OUT, "-I", HERE,
-           "-I", os.path.join(ROOT, "include"), "-Wno-unused-result", "-o", LIB] + srcs
-    r = subprocess.run(cmd, capture_output=True, text=True)
-    if r.returncode != 0:
-        sys.stderr.write(r.stdout + r.stderr)
-        raise RuntimeError("emulator build failed")
+    flags = ["-std=c++20", os.environ.get("EF_EMU_OPT", "-O1"), "-g"] + os.environ.get("EF_EMU_SAN", "").split() + [
+        "-fPIC", "-pthread"]
+    inc = ["-I", OUT, "-I", HERE, "-I", os.path.join(ROOT, "include"), "-Wno-unused-result"]
+
+    def run(cmd):
+        r = subprocess.run(cmd, capture_output=True, text=True)
+        if r.returncode != 0:
+            raise RuntimeError(f"emulator build failed: {' '.join(cmd)}\n{r.stdout}{r.stderr}")
+
+    def compile_one(src):
+        obj = os.path.join(OUT, os.path.basename(src) + ".o")
+        run([clangxx()] + flags + inc + ["-c", src, "-o", obj])
+        return obj
+
+    with concurrent.futures.ThreadPoolExecutor(max_workers=min(len(srcs), os.cpu_count() or 4)) as ex:
+        objs = list(ex.map(compile_one, srcs))
+    run([clangxx()] + flags + ["-shared", "-o", LIB + ".tmp"] + objs)
+    os.replace(LIB + ".tmp", LIB)
     return LIB
 
 
