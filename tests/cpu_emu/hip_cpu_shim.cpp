@@ -3,6 +3,7 @@
 
 #include <dlfcn.h>
 
+#include <atomic>
 #include <cstdint>
 #include <map>
 #include <mutex>
@@ -15,6 +16,23 @@ static const size_t PAGE = 4096;
 static std::map<void*, std::pair<void*, size_t>> g_maps;
 static std::map<void*, size_t> g_sizes;  // user bytes of each allocation
 static std::mutex g_mu;
+
+// What a test can ask of the emulation: graph launches, f64 16x16x4 products (waves), device
+// synchronisations (explicit ones and those a free implies) so far, and bytes allocated now.
+static std::atomic<long long> g_graph_launches{0}, g_products{0}, g_device_syncs{0};
+extern "C" long long emu_count(const char* what) {
+    const std::string w = what;
+    if (w == "graph launches") return g_graph_launches;
+    if (w == "products") return g_products;
+    if (w == "device syncs") return g_device_syncs;
+    if (w == "device bytes") {
+        std::lock_guard<std::mutex> lk(g_mu);
+        long long n = 0;
+        for (auto& m : g_sizes) n += (long long)m.second;
+        return n;
+    }
+    return -1;
+}
 
 // Each buffer sits inside its own reservation with 1 GiB of PROT_NONE on both sides, so
 // a stray access anywhere near it faults.  EF_EMU_GUARD=front aligns the buffer to the
@@ -106,7 +124,13 @@ void emu_ptrcheck(const void* p, size_t n, const char* what, const void* kernel,
     }
 }
 
+hipError_t hipDeviceSynchronize() {
+    g_device_syncs++;
+    return emu_capturing() ? hipErrorStreamCaptureUnsupported : 0;
+}
+
 hipError_t hipFree(void* p) {
+    g_device_syncs++;
     std::lock_guard<std::mutex> lk(g_mu);
     auto it = g_maps.find(p);
     if (it == g_maps.end()) { fprintf(stderr, "hipFree of unknown pointer\n"); abort(); }
@@ -141,6 +165,7 @@ emu_d4 emu_mfma_f64(double a, double b, emu_d4 c, int, int, int) {
     g_par ^= 1;
     g_mfma_a[p][t] = a;
     g_mfma_b[p][t] = b;
+    if (l == 0) g_products++;
     emu_wave_sync();
     emu_d4 out = c;
     for (int v = 0; v < 4; v++) {
@@ -255,6 +280,7 @@ hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t g, void*, char*, si
 }
 hipError_t hipGraphLaunch(hipGraphExec_t e, hipStream_t) {
     if (g_capture) return hipErrorStreamCaptureUnsupported;
+    g_graph_launches++;
     for (auto& n : e->nodes) n();
     return 0;
 }

@@ -98,7 +98,7 @@ inline hipError_t hipStreamSynchronize(hipStream_t) { return emu_capturing() ? h
 #define hipHostMallocDefault 0u
 inline hipError_t hipHostMalloc(void** p, size_t n, unsigned) { *p = std::malloc(n ? n : 1); return *p ? 0 : 2; }
 inline hipError_t hipHostFree(void* p) { std::free(p); return 0; }
-inline hipError_t hipDeviceSynchronize() { return 0; }
+hipError_t hipDeviceSynchronize();
 inline hipError_t hipFuncGetAttributes(hipFuncAttributes* a, const void*) { *a = hipFuncAttributes{}; return 0; }
 inline hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int) { return 0; }
 // device symbols are host objects here: their address is the symbol's own
