@@ -332,16 +332,20 @@ void record_end(ef_patches_s* p) {
     p->ev_recorded = true;
 }
 
-// Block-tridiagonal path: launches of up to 16 right-hand sides (the packed Neumann maps' work grows
-// with them), [rhs][patch][...] layouts throughout.
+// Block-tridiagonal path: launches of up to 16 right-hand sides, [rhs][patch][...] layouts throughout.
+// The packed Neumann maps' work grows with them: a launch takes as many as fit 256 MiB of it (8 of 4,096
+// patches of 32 x 32 cells, which keeps four to a wave), and at least one.
 // vz: work space of the packed Neumann maps, P N^2 doubles, one right-hand side per launch (null: the
 // batch's own, grown as needed).
+constexpr long long BT_WORK_DOUBLES = 1LL << 25;
 void launch_bt(ef_patches_s* p, int op, const double* g, const double* f, double* out, int nrhs, double* vz = nullptr) {
     const long long NN = (long long)p->N * p->N, B4 = 4LL * p->N;
     if (op == PATCH_OP_SOLVE && g == nullptr) throw EfError(EF_ERR_ARG, "boundary data g is required");
     const int mode = op == PATCH_OP_SOLVE ? 1 : g ? 2 : 0;
-    const int step = vz ? 1 : 16;
+    int step = vz ? 1 : 16;
     if (p->packed && op == PATCH_OP_MAP_D2N && !vz) {
+        const long long fit = BT_WORK_DOUBLES / (p->P * NN);
+        step = (int)std::min<long long>(step, std::max<long long>(fit < 4 ? fit : fit / 4 * 4, 1));
         p->vz.ensure((size_t)p->P * NN * std::min(nrhs, step));
         vz = p->vz.p;
     }

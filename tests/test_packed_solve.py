@@ -40,3 +40,32 @@ def test_packed_solve_strided(patch_ctx):
 
 def test_emu_packed_solve(emu_ctx):
     packed_case(emu_ctx, 16, 1, 5, seed=3)
+
+
+@pytest.mark.gpu
+def test_packed_work_is_bounded(patch_ctx):
+    """Neumann maps of 16 right-hand sides keep at most 256 MiB of work for a batch whose 16 would take 288."""
+    import ctypes
+    from ellipticforest_amd import _lib
+    N, P, k = 32, 2304, 16
+    tp.say(f"packed Neumann maps, {P} patches, N={N}, {k} right-hand sides: work space")
+    rng = np.random.default_rng(8)
+    bounds = tp.random_bounds(rng, P)
+    pv = _lib.Patches(patch_ctx, bounds, N, solver_type=_lib.EF_SOLVER_FIVE_POINT, cell=tp.variable_cells(bounds, N))
+    assert pv.packed
+    f = rng.standard_normal((k, P, N * N))
+    fd, hd = _lib.DeviceArray(patch_ctx, f.shape), _lib.DeviceArray(patch_ctx, (k, P, 4 * N))
+    fd.upload(f)
+
+    def free():
+        a, b = ctypes.c_size_t(), ctypes.c_size_t()
+        assert ctypes.CDLL("libamdhip64.so").hipMemGetInfo(ctypes.byref(a), ctypes.byref(b)) == 0
+        return a.value
+
+    before = free()
+    pv.apply_device(_lib.EF_PATCH_MAP_D2N, None, fd.ptr, hd.ptr, k)
+    pv.sync()
+    assert before - free() <= 260 << 20
+    h = hd.download().reshape(k, P, 4 * N)
+    for c in (0, 11, 12, 15):
+        assert np.array_equal(h[c], pv.map_d2n(None, f[c])[0]), c
