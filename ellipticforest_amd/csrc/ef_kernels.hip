@@ -345,12 +345,19 @@ __device__ inline void bt_substitute(const LeafDesc& L, int Nn, double* b, doubl
 
 // Leaf solve for every (leaf, rhs) with variable coefficients.  Modes: 0 particular
 // Neumann data (g = 0, h out), 1 solve with g (u out), 2 mapD2N with g (h out).
+// One workgroup per (leaf, rhs).  BY_LEAF: eight leaves (one per XCD, workgroups going to them in turn) times
+// all right-hand sides after one another, so that the L2 that read a leaf's factors serves its other
+// right-hand sides; otherwise all leaves of one right-hand side after one another.
+template <bool BY_LEAF>
 __global__ void __launch_bounds__(256) bt_solve_kernel(const LeafDesc* leaves, int Nn, int nleaves, int k, int mode,
                                                        const double* f, int f_zero, const double* garena,
                                                        double* harena, double* u, long long vcs) {
     __shared__ double b[BT_MAXN * BT_MAXN];
     __shared__ double tmp[BT_MAXN];
-    const int leaf = blockIdx.x, rhs = blockIdx.y;
+    const long long group = blockIdx.y + (long long)gridDim.y * blockIdx.z;  // of eight leaves
+    const int leaf = BY_LEAF ? (int)(8 * group) + (int)(blockIdx.x & 7) : (int)blockIdx.x;
+    const int rhs = BY_LEAF ? (int)(blockIdx.x >> 3) : (int)blockIdx.y;
+    if (leaf >= nleaves) return;  // uniform per workgroup
     const LeafDesc L = leaves[leaf];
     const int tid = threadIdx.x;
     const int NN = Nn * Nn;
@@ -1133,8 +1140,14 @@ void launch_bt_solve(const LeafDesc* leaves, int Nn, int nleaves, int k, int mod
     else if (Nn == 32)
         hipLaunchKernelGGL(bt_solve_wave_kernel<32>, dim3(blocks), dim3(256), 0, s, leaves, nleaves, k, mode, f,
                            f_zero, garena, harena, u, vcs);
-    else
-        hipLaunchKernelGGL(bt_solve_kernel, dim3(nleaves, k), dim3(256), 0, s, leaves, Nn, nleaves, k, mode, f, f_zero,
+    else if (k > 1 && Nn >= 8) {
+        // the factors are N / 2 times the load and the solution: right-hand side after right-hand side, 2,000 patches
+        // of 24^2 took 3,119 us at k = 16 (20^2 1,939, 12^2 680), so 2,276 (1,584, 527); of 6^2 177, so 199
+        const unsigned groups = (unsigned)(nleaves + 7) / 8, gy = std::min(groups, 65535u);
+        hipLaunchKernelGGL(bt_solve_kernel<true>, dim3(8 * k, gy, (groups + gy - 1) / gy), dim3(256), 0, s, leaves, Nn,
+                           nleaves, k, mode, f, f_zero, garena, harena, u, vcs);
+    } else
+        hipLaunchKernelGGL(bt_solve_kernel<false>, dim3(nleaves, k), dim3(256), 0, s, leaves, Nn, nleaves, k, mode, f, f_zero,
                            garena, harena, u, vcs);
 }
 

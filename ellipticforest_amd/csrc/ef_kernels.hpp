@@ -13,6 +13,7 @@ __global__ void bt_factor_wave_kernel(const LeafDesc* leaves, int nleaves);
 // five-point matrix is diagonally dominant (cells_dominant), so the wave kernel may skip the
 // pivot search.
 void launch_bt_factor(const LeafDesc* leaves, int Nn, int nleaves, hipStream_t s, bool dominant = false);
+template <bool BY_LEAF>
 __global__ void bt_solve_kernel(const LeafDesc* leaves, int Nn, int nleaves, int k, int mode, const double* f,
                                 int f_zero, const double* garena, double* harena, double* u, long long vcs);
 __global__ void bt_dtn_kernel(const LeafDesc* leaves, int Nn, int first, double* work);
