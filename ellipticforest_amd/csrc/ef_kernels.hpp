@@ -47,7 +47,7 @@ constexpr int BT_MAX_N = 32;  // largest leaf side of the block-tridiagonal path
 template <int NB, bool FULL, int OP, int NV = 0>
 __global__ void patch_fd_kernel(PatchFDArgs p, const int* __restrict__ cls, const PatchCoef* __restrict__ coef,
                                 const long long* __restrict__ g_off, const long long* __restrict__ h_off);
-template <int STAGE>
+template <int STAGE, bool SPLIT>
 __global__ void patch_large_gemm_kernel(PatchLargeArgs a);
 __global__ void patch_large_out_kernel(PatchLargeArgs a);
 __global__ void fill_kernel(double* p, double v, long long n);

@@ -252,6 +252,22 @@ void launch_fd(ef_patches_s* p, int op, const double* g, const double* f, double
     efk::launch_patch_fd(a, p->NB, p->max_blocks, p->stream);
 }
 
+// The four products of the items of `a`; the last one of Neumann data on the blocks of the edge cells only.
+template <bool SPLIT>
+void large_products(const PatchLargeArgs& a, hipStream_t s) {
+    const int tn = ((a.N + 15) / 16 + 1) / 2, edge = 4 * tn - 4;
+    auto blocks = [&](int n) { return dim3((unsigned)(SPLIT ? n : (n + 3) / 4), (unsigned)a.items); };
+    const dim3 block(256), grid = blocks(tn * tn), last = blocks(a.op == PATCH_OP_SOLVE ? tn * tn : edge);
+    hipLaunchKernelGGL((patch_large_gemm_kernel<0, SPLIT>), grid, block, 0, s, a);
+    EF_LAUNCH_CHECK();
+    hipLaunchKernelGGL((patch_large_gemm_kernel<1, SPLIT>), grid, block, 0, s, a);
+    EF_LAUNCH_CHECK();
+    hipLaunchKernelGGL((patch_large_gemm_kernel<2, SPLIT>), grid, block, 0, s, a);
+    EF_LAUNCH_CHECK();
+    hipLaunchKernelGGL((patch_large_gemm_kernel<3, SPLIT>), last, block, 0, s, a);
+    EF_LAUNCH_CHECK();
+}
+
 // Large patches: chunks of items through the four products and, for Neumann data, the edge cells.
 // W1, W2: work buffers of at least wcap doubles each (null: the batch's own, grown as needed).
 // Items are independent, so the chunking does not change any result.
@@ -291,16 +307,11 @@ void launch_large(ef_patches_s* p, int op, const double* g, const double* f, dou
         a.W2 = W2;
         a.out = out;
         a.item0 = (op == PATCH_OP_DTN) ? 0 : first;
-        const int tn = (Np + 31) / 32;
-        const dim3 grid((unsigned)(tn * tn), (unsigned)items), block(256);
-        hipLaunchKernelGGL(patch_large_gemm_kernel<0>, grid, block, 0, p->stream, a);
-        EF_LAUNCH_CHECK();
-        hipLaunchKernelGGL(patch_large_gemm_kernel<1>, grid, block, 0, p->stream, a);
-        EF_LAUNCH_CHECK();
-        hipLaunchKernelGGL(patch_large_gemm_kernel<2>, grid, block, 0, p->stream, a);
-        EF_LAUNCH_CHECK();
-        hipLaunchKernelGGL(patch_large_gemm_kernel<3>, grid, block, 0, p->stream, a);
-        EF_LAUNCH_CHECK();
+        // sides up to 64 have four 32 x 32 blocks of 3 or 4 blocks of k: from a block per SIMD on a wave takes one
+        // whole (2,000 patches of 48^2: 182 us with the k range split over a workgroup, 134 so; 256 of 33^2: 48
+        // and 43; 128 of 33^2: 35 and 41).  Of the larger sides 96^2 loses 10 % by it at 2,000 patches, 112^2 gains 6 %.
+        if (Np <= 64 && 4LL * items >= 1024) large_products<false>(a, p->stream);
+        else large_products<true>(a, p->stream);
         if (op == PATCH_OP_SOLVE) continue;
         hipLaunchKernelGGL(patch_large_out_kernel, dim3(blocks_for((long long)items * 4 * N)), dim3(256), 0, p->stream, a);
         EF_LAUNCH_CHECK();
