@@ -1735,7 +1735,10 @@ __global__ void __launch_bounds__(256) tree_root_robin_kernel(const double* T, c
     auto scale = [&](int i) {
         auto fine = [](double x) { return fabs(x) > 1e-150 && fabs(x) < 1e150; };
         const double t = T[(long long)i * m + i];
-        if (fine(b[i])) return ldexp(1.0, -ilogb(b[i]));
+        if (fine(b[i])) {  // (an a / b beyond the range leaves the row as it is)
+            const double f = ldexp(1.0, -ilogb(b[i]));
+            return fabs(a[i]) * f < 1e150 ? f : 1.0;
+        }
         return b[i] == 0.0 && fine(a[i]) && fine(t) ? ldexp(1.0, ilogb(t) - ilogb(a[i])) : 1.0;
     };
     if (e < nA) {
