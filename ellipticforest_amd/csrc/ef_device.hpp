@@ -31,13 +31,17 @@ namespace efk {
 // global address space (device compilation only; the host pass never dereferences them).
 #if defined(__HIP_DEVICE_COMPILE__)
 #define EF_GLOBAL __attribute__((address_space(1)))
+#define EF_CONSTANT __attribute__((address_space(4)))
 #else
 #define EF_GLOBAL
+#define EF_CONSTANT
 #endif
 template <class T>
 __host__ __device__ inline const EF_GLOBAL T* gmem(const T* p) { return (const EF_GLOBAL T*)p; }
 template <class T>
 __host__ __device__ inline EF_GLOBAL T* gmem(T* p) { return (EF_GLOBAL T*)p; }
+// A word that no kernel in flight needs the newest value of, uniform over the launch: a scalar load.
+__host__ __device__ inline int cmem(const int* p) { return *(const EF_CONSTANT int*)p; }
 
 enum Side { W = 0, E = 1, S = 2, N = 3 };
 

@@ -6,7 +6,7 @@
 // The reference forms X, S_RHS and H element by element, calls dgesv for S = X^-1 S_RHS and
 // dgemm for T = blkdiag + H S (Matrix.hpp:827-953), one family at a time.  Here:
 //  * X is inverted once per merge (blocked Gauss-Jordan in natural order with the multipliers
-//    checked, redone with partial pivoting where one is large; every O(m^3) step a batched
+//    checked, going on with partial pivoting where one is large; every O(m^3) step a batched
 //    MFMA product), so the upward sweep's mergeW_ is a product with X^-1 instead of a
 //    re-factorisation per solve;
 //  * S = X^-1 S_RHS and T = blkdiag + H S read S_RHS and H straight out of the children's
@@ -993,25 +993,23 @@ __global__ void __launch_bounds__(256) gj_update_kernel(GJArgs a) {
             }
 }
 
-// Column order of the inverse: the interchanges undone from the last to the first.
+// Column order of the inverse: the interchanges undone from the last to the first, column k's.  Each entry is followed
+// through them by a thread of its own (the last one undone is the first it meets): one thread exchanging
+// entries in LDS took 66 us for m = 1024, so 28.
 __global__ void __launch_bounds__(256) gj_perm_kernel(GJArgs a) {
-    __shared__ int idx[GJ_MAXM];
-    const int b = blockIdx.x, tid = threadIdx.x, m = a.m;
-    for (int i = tid; i < m; i += 256) idx[i] = i;
+    __shared__ int piv[GJ_MAXM];
+    const int b = blockIdx.y, tid = threadIdx.x, m = a.m;
+    const int* ipiv = a.ipiv + (long long)b * m;
+    for (int i = a.k + tid; i < m; i += 256) piv[i] = min(max(ipiv[i], 0), m - 1);
     __syncthreads();
-    if (tid == 0) {
-        const int* ipiv = a.ipiv + (long long)b * m;
-        for (int c = m - 1; c >= 0; c--) {
-            const int p = min(max(ipiv[c], 0), m - 1);
-            if (p != c) {
-                const int t = idx[c];
-                idx[c] = idx[p];
-                idx[p] = t;
-            }
-        }
+    const int i = (int)blockIdx.x * 256 + tid;
+    int x = i;
+#pragma unroll 8
+    for (int c = a.k; c < m; c++) {
+        const int p = piv[c];
+        x = x == c ? p : x == p ? c : x;
     }
-    __syncthreads();
-    for (int i = tid; i < m; i += 256) a.src[(long long)b * m + i] = idx[i];
+    if (i < m) a.src[(long long)b * m + i] = x;
 }
 
 // X^-1(i, j) = W(i, idx(j)), written to the operator arena.
@@ -1031,8 +1029,8 @@ __global__ void __launch_bounds__(256) gj_gather_kernel(GJArgs a) {
 // boundary operators), so Gauss-Jordan needs no pivot search on them: over adaptive, variable and
 // uniform meshes with lambda <= 0 the largest multiplier is 1.3, and the inverse's residual equals
 // a pivoted LU's.  These kernels eliminate in natural order and check every multiplier against
-// INV_LMAX; one beyond it (an indefinite system, a zero pivot, a NaN) sets *flag, and the caller
-// inverts again with the pivoted kernels above.  What bounds the pivoted path is its 32-column panel,
+// INV_LMAX; one beyond it (an indefinite system, a zero pivot, a NaN) stops the elimination, and the
+// caller goes on with the pivoted kernels above from the column it stopped at.  What bounds the pivoted path is its 32-column panel,
 // a chain of 32 dependent column searches (52 us per launch): the inversions of the adaptive
 // Poisson mesh (1,937 merges, m = 64 .. 1024) took 7.4 ms of GPU time with it and take 1.2 ms so,
 // those of 1,024 leaves of 32 x 32 cells 12.9 and 2.3 ms.
@@ -1044,6 +1042,11 @@ __device__ inline int formed_here(int x) {
 #endif
     return x;
 }
+
+// Step k has met a large multiplier: no step of the launch sequence from k on is taken (inv_stopped), so
+// the matrices stay as they were before it.  Of a batch, the first such step counts.
+__device__ inline void inv_stop(int* stop, int k) { atomicMax(stop, INV_STOP - k); }
+__device__ inline bool inv_stopped(int stop, int k) { return stop >= INV_STOP - k; }
 
 // 1 / x: hardware estimate and two Newton steps (relative error about 1 ulp; inf or NaN at 0)
 __device__ inline double inv_rcp(double x) {
@@ -1121,6 +1124,7 @@ template <int MT, int WAVES>
 struct InvShared {
     double rp[2][MT][4][64];
     alignas(16) double tr[WAVES][16 * 18];
+    int bad[2];  // a multiplier of an even, an odd step was too large
 };
 
 // In-place inversion of mt x mt tiles of 16 x 16 (mt <= MT <= WAVES): wave w holds tile row w, tile
@@ -1160,6 +1164,7 @@ __device__ inline void inv_tiles(td4 (&T)[MT], int mt, InvShared<MT, WAVES>& sh,
                 for (int v = 0; v < 4; v++) sh.rp[k & 1][j][v][lane] = T[j][v];
     };
     if (wave == 0) {
+        sh.bad[lane & 1] = 0;
         inv16(T[0], tr, ok, [](int) {});
         publish(0);
     }
@@ -1175,6 +1180,8 @@ __device__ inline void inv_tiles(td4 (&T)[MT], int mt, InvShared<MT, WAVES>& sh,
 #pragma unroll
         for (int s = 0; s < 4; s++) a[s] = tr[r * 18 + 4 * s + q];
         __syncthreads();
+        // the step before (a step's word is next written two barriers on)
+        if (!OVERLAP && kb > 0 && sh.bad[(kb - 1) & 1]) break;  // uniform per workgroup
         const double (&rp)[MT][4][64] = sh.rp[kb & 1];
         if (wave == kb) {
 #pragma unroll
@@ -1232,6 +1239,7 @@ __device__ inline void inv_tiles(td4 (&T)[MT], int mt, InvShared<MT, WAVES>& sh,
                 put(kb, L);
             }
         }
+        if (!OVERLAP && __ballot(!ok)) sh.bad[kb & 1] = 1;
     }
 }
 
@@ -1241,7 +1249,7 @@ __device__ inline void inv_tiles(td4 (&T)[MT], int mt, InvShared<MT, WAVES>& sh,
 // for the registers, the adaptive Poisson mesh's matrices of order 64 took 140 us, so 85 us.
 template <int MT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8)))
-inv_wave_kernel(const double* __restrict__ A, double* __restrict__ Ai, int m, int B, int* flag) {
+inv_wave_kernel(const double* __restrict__ A, double* __restrict__ Ai, int m, int B, int* stop) {
     __shared__ __attribute__((aligned(16))) double tr_all[4][16 * 18];
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     const int q = lane >> 4, r = lane & 15, b = (int)blockIdx.x * 4 + wave;
@@ -1305,6 +1313,7 @@ inv_wave_kernel(const double* __restrict__ A, double* __restrict__ Ai, int m, in
             for (int s = 0; s < 4; s++) x = mfma_f64(a[s], T[kb][j][s], x);
             T[kb][j] = x;
         }
+        if (__ballot(!ok)) break;
     }
     const int ms = formed_here(m);  // the stores' addresses are not kept from the loads
     auto* Ib = gmem(Ai) + (long long)b * ms * ms + r;
@@ -1317,7 +1326,7 @@ inv_wave_kernel(const double* __restrict__ A, double* __restrict__ Ai, int m, in
             for (int j = 0; j < MT; j++)
                 if (row < ms && 16 * j + r < ms) Ib[(long long)row * ms + 16 * j] = T[i][j][v];
         }
-    if (!ok) *flag = 1;
+    if (!ok) inv_stop(stop, 0);
 }
 
 template __global__ void inv_wave_kernel<1>(const double*, double*, int, int, int*);
@@ -1328,7 +1337,7 @@ template __global__ void inv_wave_kernel<4>(const double*, double*, int, int, in
 template <int MT>
 __global__ void __launch_bounds__(64 * MT) __attribute__((amdgpu_waves_per_eu(2, 8)))
 inv_small_kernel(const double* __restrict__ A, double* __restrict__ Ai, int m,
-                                                            int* flag) {
+                                                            int* stop) {
     __shared__ InvShared<MT, MT> sh;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     const int q = lane >> 4, r = lane & 15, mt = (m + 15) / 16;
@@ -1357,7 +1366,7 @@ inv_small_kernel(const double* __restrict__ A, double* __restrict__ Ai, int m,
         for (int j = 0; j < MT; j++)
             if (row < ms && 16 * j + r < ms) p[16 * j] = T[j][v];
     }
-    if (!ok) *flag = 1;
+    if (!ok) inv_stop(stop, 0);
 }
 
 template __global__ void inv_small_kernel<8>(const double*, double*, int, int*);
@@ -1369,8 +1378,9 @@ template __global__ void inv_small_kernel<8>(const double*, double*, int, int*);
 // m <= 1024.  Inverting the pivot block in every workgroup of the multipliers instead, with the
 // inversion in the open, took 24 + 8 us.
 
-// P^-1 of the pivot block (nb x nb, here in strips of tiles), zero beyond nb, into Pn (INV_NB x INV_NB)
-__device__ inline void inv_pivot_block(td4 (&T)[INV_NB / 16], int nb, InvShared<INV_NB / 16, 4>& sh, double* Pn, int* flag) {
+// P^-1 of step k's pivot block (nb x nb, here in strips of tiles), zero beyond nb, into Pn (INV_NB x INV_NB)
+__device__ inline void inv_pivot_block(td4 (&T)[INV_NB / 16], int nb, InvShared<INV_NB / 16, 4>& sh, double* Pn, int k,
+                                       int* stop) {
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     const int q = lane >> 4, r = lane & 15;
     bool ok = true;
@@ -1382,12 +1392,12 @@ __device__ inline void inv_pivot_block(td4 (&T)[INV_NB / 16], int nb, InvShared<
             const int row = 16 * wave + 4 * v + q, col = 16 * j + r;
             gmem(Pn)[row * INV_NB + col] = (row < nb && col < nb) ? T[j][v] : 0.0;
         }
-    if (!ok) *flag = 1;
+    if (!ok) inv_stop(stop, k);
 }
 
 // the first step's pivot block, one workgroup per matrix
 __global__ void __launch_bounds__(256) inv_pivot_kernel(const double* __restrict__ A, double* __restrict__ Pn, int m,
-                                                        int* flag) {
+                                                        int* stop) {
     __shared__ InvShared<INV_NB / 16, 4> sh;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     const int q = lane >> 4, r = lane & 15;
@@ -1398,14 +1408,15 @@ __global__ void __launch_bounds__(256) inv_pivot_kernel(const double* __restrict
 #pragma unroll
         for (int v = 0; v < 4; v++)  // m > INV_NB
             T[j][v] = Ab[(long long)(16 * wave + 4 * v + q) * m + 16 * j + r];
-    inv_pivot_block(T, INV_NB, sh, Pn + (long long)blockIdx.x * INV_NB * INV_NB, flag);
+    inv_pivot_block(T, INV_NB, sh, Pn + (long long)blockIdx.x * INV_NB * INV_NB, 0, stop);
 }
 
 // M = P^-1 on the pivot rows, -A P^-1 elsewhere (zero beyond the matrix's columns): one wave per
 // 16 rows x 32 columns, all operands loaded before the products.
 __global__ void __launch_bounds__(512) inv_mult_kernel(const double* __restrict__ A, double* __restrict__ Mm,
-                                                       const double* __restrict__ Pn, int m, int k, int* flag) {
+                                                       const double* __restrict__ Pn, int m, int k, int* stop) {
     constexpr int MT = INV_NB / 16;
+    const int st = cmem(stop);  // (what this launch itself finds is for the next one)
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     const int q = lane >> 4, r = lane & 15;
     const int nb = min(INV_NB, m - k), row0 = (int)blockIdx.x * 64 + 16 * (wave & 3), j0 = 2 * (wave >> 2);
@@ -1419,6 +1430,7 @@ __global__ void __launch_bounds__(512) inv_mult_kernel(const double* __restrict_
         for (int j = 0; j < 2; j++)
 #pragma unroll
             for (int v = 0; v < 4; v++) x[j][v] = Pb[(row0 - k + 4 * v + q) * INV_NB + 16 * (j0 + j) + r];
+        if (inv_stopped(st, k)) return;
     } else {
         // lane group q takes columns 16 t + 4q + s at step s; m, nb are multiples of 4
         td2 a[MT][2];
@@ -1436,6 +1448,7 @@ __global__ void __launch_bounds__(512) inv_mult_kernel(const double* __restrict_
             for (int j = 0; j < 2; j++)
 #pragma unroll
                 for (int s = 0; s < 4; s++) b[t][j][s] = Pb[(16 * t + 4 * q + s) * INV_NB + 16 * (j0 + j) + r];
+        if (inv_stopped(st, k)) return;  // (after the loads are issued: the wait for it is theirs)
         x[0] = x[1] = td4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
         for (int t = 0; t < MT; t++)
@@ -1448,7 +1461,7 @@ __global__ void __launch_bounds__(512) inv_mult_kernel(const double* __restrict_
         for (int j = 0; j < 2; j++)
 #pragma unroll
             for (int v = 0; v < 4; v++) ok = ok & (fabs(x[j][v]) <= INV_LMAX);
-        if (!ok) *flag = 1;
+        if (!ok) inv_stop(stop, k);
     }
 #pragma unroll
     for (int j = 0; j < 2; j++)
@@ -1466,8 +1479,9 @@ __global__ void __launch_bounds__(512) inv_mult_kernel(const double* __restrict_
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8)))
 inv_update_kernel(const double* __restrict__ Wa, double* __restrict__ Wb,
                                                          const double* __restrict__ Mm, double* __restrict__ Pn, int m,
-                                                         int k, int* flag) {
+                                                         int k, int* stop) {
     constexpr int MT = INV_NB / 16;
+    const int st = cmem(stop);  // (what this launch itself finds is for the next one)
     __shared__ union {
         InvShared<MT, 4> inv;
         double blk[MT][MT][4][64];  // the next pivot block, from the waves' quarters to their strips
@@ -1492,6 +1506,7 @@ inv_update_kernel(const double* __restrict__ Wa, double* __restrict__ Wb,
 #pragma unroll
                 for (int v = 0; v < 4; v++)
                     acc[i][j][v] = Mb[(long long)min(row0 + 16 * i + 4 * v + q, m - 1) * INV_NB + col0 - k + 16 * j + r];
+        if (inv_stopped(st, k)) return;
     } else {
         const bool pivot_rows = (t / tpr) * 64 == k;
         const int c0 = min(col0 + r, m - 1), c1 = min(col0 + 16 + r, m - 1);
@@ -1506,26 +1521,29 @@ inv_update_kernel(const double* __restrict__ Wa, double* __restrict__ Wb,
             }
         const auto* m0 = Mb + (long long)min(row0 + r, m - 1) * INV_NB;
         const auto* m1 = Mb + (long long)min(row0 + 16 + r, m - 1) * INV_NB;
+        double a0[MT][4], a1[MT][4], b0[MT][4], b1[MT][4];
 #pragma unroll
-        for (int kb = 0; kb < INV_NB; kb += 16) {
-            const int k0 = kb + 4 * q;  // lane group q takes k = kb + 4q + s at step s
-            double a0[4], a1[4], b0[4], b1[4];
+        for (int t4 = 0; t4 < MT; t4++) {
+            const int k0 = 16 * t4 + 4 * q;  // lane group q takes k = 16 t4 + 4q + s at step s
 #pragma unroll
             for (int s = 0; s < 4; s++) {
-                a0[s] = m0[k0 + s];
-                a1[s] = m1[k0 + s];
+                a0[t4][s] = m0[k0 + s];
+                a1[t4][s] = m1[k0 + s];
                 const auto* brow = Ab + (long long)(k + min(k0 + s, nb - 1)) * m;  // past nb: times a zero
-                b0[s] = brow[c0];
-                b1[s] = brow[c1];
-            }
-#pragma unroll
-            for (int s = 0; s < 4; s++) {
-                acc[0][0] = mfma_f64(a0[s], b0[s], acc[0][0]);
-                acc[0][1] = mfma_f64(a0[s], b1[s], acc[0][1]);
-                acc[1][0] = mfma_f64(a1[s], b0[s], acc[1][0]);
-                acc[1][1] = mfma_f64(a1[s], b1[s], acc[1][1]);
+                b0[t4][s] = brow[c0];
+                b1[t4][s] = brow[c1];
             }
         }
+        if (inv_stopped(st, k)) return;
+#pragma unroll
+        for (int t4 = 0; t4 < MT; t4++)
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                acc[0][0] = mfma_f64(a0[t4][s], b0[t4][s], acc[0][0]);
+                acc[0][1] = mfma_f64(a0[t4][s], b1[t4][s], acc[0][1]);
+                acc[1][0] = mfma_f64(a1[t4][s], b0[t4][s], acc[1][0]);
+                acc[1][1] = mfma_f64(a1[t4][s], b1[t4][s], acc[1][1]);
+            }
     }
 #pragma unroll
     for (int i = 0; i < 2; i++)
@@ -1536,7 +1554,7 @@ inv_update_kernel(const double* __restrict__ Wa, double* __restrict__ Wb,
                 const int row = row0 + 16 * i + 4 * v + q, col = col0 + 16 * j + r;
                 if (row < m && col < m) Bb[(long long)row * m + col] = acc[i][j][v];
             }
-    if (kn >= m || blockIdx.x != 0) return;  // uniform per workgroup
+    if (kn >= m || blockIdx.x != 0) return;  // uniform per workgroup (st is too: step k's stop is older than this launch)
     const int nn = min(INV_NB, m - kn);
 #pragma unroll
     for (int i = 0; i < 2; i++)
@@ -1555,7 +1573,7 @@ inv_update_kernel(const double* __restrict__ Wa, double* __restrict__ Wb,
             T[j][v] = (row < nn && col < nn) ? x : (row == col ? 1.0 : 0.0);
         }
     __syncthreads();
-    inv_pivot_block(T, nn, sh.inv, Pn + (long long)blockIdx.y * INV_NB * INV_NB, flag);
+    inv_pivot_block(T, nn, sh.inv, Pn + (long long)blockIdx.y * INV_NB * INV_NB, kn, stop);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1912,7 +1930,7 @@ size_t gj_work_ints(int m, int B) {
     return (size_t)B * ((size_t)GJ_MAXCH * GJ_NB + GJ_NB + 2 * (size_t)m + GJ_NB);
 }
 
-void run_gj_inverse(double* wa, double* xi, int m, int B, const GJWork& w, int* info, hipStream_t s) {
+void run_gj_inverse(double* wa, double* xi, int m, int B, const GJWork& w, int* info, hipStream_t s, int k0) {
     if (B <= 0) return;
     if (m < 1 || m > GJ_MAXM)
         throw EfError(EF_ERR_ARG, "interface system of order " + std::to_string(m) + " exceeds the inversion limit " +
@@ -1936,7 +1954,7 @@ void run_gj_inverse(double* wa, double* xi, int m, int B, const GJWork& w, int* 
     double* cur = wa;
     double* nxt = w.wb;
     const int tpr = (m + 31) / 32;
-    for (int k = 0; k < m; k += GJ_NB) {
+    for (int k = k0; k < m; k += GJ_NB) {
         a.Wa = cur; a.Wb = nxt; a.k = k;
         a.nch = (m - k + GJ_CH - 1) / GJ_CH;
         const int rows = m - k;
@@ -1957,8 +1975,8 @@ void run_gj_inverse(double* wa, double* xi, int m, int B, const GJWork& w, int* 
         EF_LAUNCH("gj_update_kernel", gj_update_kernel, dim3(blocks_for((long long)tpr * tpr, 4), B), dim3(256), s, a);
         std::swap(cur, nxt);
     }
-    a.Wa = cur; a.Wb = nxt; a.k = 0;
-    EF_LAUNCH("gj_perm_kernel", gj_perm_kernel, dim3(B), dim3(256), s, a);
+    a.Wa = cur; a.Wb = nxt; a.k = k0;
+    EF_LAUNCH("gj_perm_kernel", gj_perm_kernel, dim3(blocks_for(m), B), dim3(256), s, a);
     EF_LAUNCH("gj_gather_kernel", gj_gather_kernel, dim3(blocks_for((long long)m * m), B), dim3(256), s, a);
 }
 
@@ -1966,7 +1984,7 @@ size_t inv_work_doubles(int m, int B) {
     return m <= INV_SMALL ? 0 : (size_t)B * ((size_t)m * m + (size_t)m * INV_NB + (size_t)INV_NB * INV_NB);
 }
 
-void run_inverse(double* wa, double* xi, int m, int B, double* work, int* flag, hipStream_t s) {
+void run_inverse(double* wa, double* xi, int m, int B, double* work, int* stop, hipStream_t s) {
     if (B <= 0) return;
     if (m < 1 || m > GJ_MAXM)
         throw EfError(EF_ERR_ARG, "interface system of order " + std::to_string(m) + " exceeds the inversion limit " +
@@ -1974,16 +1992,16 @@ void run_inverse(double* wa, double* xi, int m, int B, double* work, int* flag, 
     const size_t mm = (size_t)m * m * B;
     check_range(wa, mm * 8, "matrices to invert");
     check_range(xi, mm * 8, "inverse output");
-    check_range(flag, sizeof(int), "inversion flag");
+    check_range(stop, sizeof(int), "inversion stop");
     // up to 64 one wave holds the matrix (128 registers a lane), up to 128 a workgroup of eight
     if (m <= 16)
-        EF_LAUNCH("inv_wave_kernel<1>", inv_wave_kernel<1>, dim3((B + 3) / 4), dim3(256), s, (const double*)wa, xi, m, B, flag);
+        EF_LAUNCH("inv_wave_kernel<1>", inv_wave_kernel<1>, dim3((B + 3) / 4), dim3(256), s, (const double*)wa, xi, m, B, stop);
     else if (m <= 32)
-        EF_LAUNCH("inv_wave_kernel<2>", inv_wave_kernel<2>, dim3((B + 3) / 4), dim3(256), s, (const double*)wa, xi, m, B, flag);
+        EF_LAUNCH("inv_wave_kernel<2>", inv_wave_kernel<2>, dim3((B + 3) / 4), dim3(256), s, (const double*)wa, xi, m, B, stop);
     else if (m <= 64)
-        EF_LAUNCH("inv_wave_kernel<4>", inv_wave_kernel<4>, dim3((B + 3) / 4), dim3(256), s, (const double*)wa, xi, m, B, flag);
+        EF_LAUNCH("inv_wave_kernel<4>", inv_wave_kernel<4>, dim3((B + 3) / 4), dim3(256), s, (const double*)wa, xi, m, B, stop);
     else if (m <= INV_SMALL)
-        EF_LAUNCH("inv_small_kernel<8>", inv_small_kernel<8>, dim3(B), dim3(512), s, (const double*)wa, xi, m, flag);
+        EF_LAUNCH("inv_small_kernel<8>", inv_small_kernel<8>, dim3(B), dim3(512), s, (const double*)wa, xi, m, stop);
     else {
         check_range(work, inv_work_doubles(m, B) * 8, "inversion work");
         if (m % 4 != 0) throw EfError(EF_ERR_INTERNAL, "inversion of an order that is not a multiple of 4");
@@ -1992,16 +2010,20 @@ void run_inverse(double* wa, double* xi, int m, int B, double* work, int* flag, 
         double* cur = wa;
         double* nxt = work;
         const int tpr = (m + 63) / 64;
-        EF_LAUNCH("inv_pivot_kernel", inv_pivot_kernel, dim3(B), dim3(256), s, (const double*)cur, Pn, m, flag);
+        EF_LAUNCH("inv_pivot_kernel", inv_pivot_kernel, dim3(B), dim3(256), s, (const double*)cur, Pn, m, stop);
         for (int k = 0; k < m; k += INV_NB) {
             double* out = (k + INV_NB >= m) ? xi : nxt;  // the last step writes the inverse where it belongs
             EF_LAUNCH("inv_mult_kernel", inv_mult_kernel, dim3(tpr, B), dim3(512), s, (const double*)cur, Mm,
-                      (const double*)Pn, m, k, flag);
+                      (const double*)Pn, m, k, stop);
             EF_LAUNCH("inv_update_kernel", inv_update_kernel, dim3(tpr * tpr, B), dim3(256), s, (const double*)cur, out,
-                      (const double*)Mm, Pn, m, k, flag);
+                      (const double*)Mm, Pn, m, k, stop);
             std::swap(cur, nxt);
         }
     }
 }
+
+int inv_stop_column(int stop, int m) { return stop == 0 ? m : INV_STOP - stop; }
+
+double* inv_state(double* wa, double* work, int k) { return k / INV_NB % 2 ? work : wa; }
 
 }  // namespace efk

@@ -153,27 +153,28 @@ __global__ void gj_gather_kernel(GJArgs a);
 
 // ---------------------------------------------------------------------------------------
 // Inversion of a batch of equally sized matrices by Gauss-Jordan in natural order (no row
-// exchanges): in registers, one workgroup per matrix, up to INV_SMALL; beyond it INV_NB columns
-// per step (mult, update) between two buffers.  A multiplier beyond INV_LMAX (or a NaN) sets the
-// flag: the result is then not to be used.  4 is three times the largest multiplier of the
+// exchanges): in registers, one wave per matrix of order <= 64 and one workgroup up to INV_SMALL; beyond
+// it INV_NB columns per step (mult, update) between two buffers.  A multiplier beyond INV_LMAX (or a
+// NaN) stops it: *stop becomes INV_STOP less the step's first column (the matrices in registers: 0), and
+// from that step on nothing is written but the multipliers.  4 is three times the largest multiplier of the
 // definite systems measured (1.3) and keeps the growth of an indefinite one that passes small.
 // ---------------------------------------------------------------------------------------
 constexpr int INV_SMALL = 128;
 constexpr int INV_NB = 64;
 constexpr double INV_LMAX = 4.0;
+constexpr int INV_STOP = 1 << 20;  // beyond every column
 
 template <int MT>
-__global__ void inv_wave_kernel(const double* A, double* Ai, int m, int B, int* flag);
+__global__ void inv_wave_kernel(const double* A, double* Ai, int m, int B, int* stop);
 template <int MT>
-__global__ void inv_small_kernel(const double* A, double* Ai, int m, int* flag);
-__global__ void inv_pivot_kernel(const double* A, double* Pn, int m, int* flag);
-__global__ void inv_mult_kernel(const double* A, double* Mm, const double* Pn, int m, int k, int* flag);
-__global__ void inv_update_kernel(const double* Wa, double* Wb, const double* Mm, double* Pn, int m, int k, int* flag);
+__global__ void inv_small_kernel(const double* A, double* Ai, int m, int* stop);
+__global__ void inv_pivot_kernel(const double* A, double* Pn, int m, int* stop);
+__global__ void inv_mult_kernel(const double* A, double* Mm, const double* Pn, int m, int k, int* stop);
+__global__ void inv_update_kernel(const double* Wa, double* Wb, const double* Mm, double* Pn, int m, int k, int* stop);
 
 // ---------------------------------------------------------------------------------------
 // Merge assembly (createMatrixBlocks_ + mergeX_, HPSAlgorithm.hpp:799-895): from the
-// four children's DtN maps (each 4n x 4n, coarsened), X (4n x 4n) into the inversion work
-// buffer and T (8n x 8n, WESN rows and columns) = diag blocks T_c(tau side, tau side).
+// four children's DtN maps (each 4n x 4n, coarsened), X (4n x 4n) into the inversion work buffer.
 // ---------------------------------------------------------------------------------------
 struct AsmDesc {
     const double* Tc[4];
@@ -243,12 +244,16 @@ struct GJWork {
 };
 size_t gj_work_doubles(int m, int B);  // doubles of wb + Pinv + Mm
 size_t gj_work_ints(int m, int B);     // ints of cand + src + ipiv + prow
-void run_gj_inverse(double* wa, double* xi, int m, int B, const GJWork& w, int* info, hipStream_t s);
+// From column k0 on (a multiple of GJ_NB): the columns before it have been eliminated in natural order.
+void run_gj_inverse(double* wa, double* xi, int m, int B, const GJWork& w, int* info, hipStream_t s, int k0 = 0);
 
 // Inversion in natural order of `B` matrices of order m held in wa (B x m x m, destroyed beyond
-// INV_SMALL); X^-1 into xi.  work: inv_work_doubles(m, B); *flag is set when a multiplier was too
-// large (never cleared here).
+// INV_SMALL); X^-1 into xi.  work: inv_work_doubles(m, B); *stop (0 before) is set when a multiplier
+// was too large: the matrices are then in inv_state(wa, work, k), the columns before k =
+// inv_stop_column(*stop, m) eliminated (k = m: none was too large), for run_gj_inverse to go on with.
 size_t inv_work_doubles(int m, int B);
-void run_inverse(double* wa, double* xi, int m, int B, double* work, int* flag, hipStream_t s);
+void run_inverse(double* wa, double* xi, int m, int B, double* work, int* stop, hipStream_t s);
+int inv_stop_column(int stop, int m);
+double* inv_state(double* wa, double* work, int k);
 
 }  // namespace efk

@@ -201,6 +201,12 @@ inline double __builtin_amdgcn_rcp(double x) { return 1.0 / x; }
 #define __builtin_amdgcn_wave_barrier() emu_wave_sync()
 // memory fences: the emulated lanes share the host's coherent memory; ordering between lanes
 // comes from the wave and block barriers
+inline int atomicMax(int* p, int v) {
+    std::atomic_ref<int> a(*p);
+    int old = a.load();
+    while (old < v && !a.compare_exchange_weak(old, v)) {}
+    return old;
+}
 #define __builtin_amdgcn_fence(order, scope) std::atomic_thread_fence(std::memory_order_seq_cst)
 // instruction-scheduling fence of the GPU compiler: nothing to do on the CPU
 #define __builtin_amdgcn_sched_barrier(mask) ((void)(mask))
