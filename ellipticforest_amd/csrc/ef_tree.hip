@@ -353,7 +353,7 @@ template __global__ void tree_gemm_kernel<2, 2, true>(const TreeGemm*, const int
 // (62; the card's large matrix product reaches 72); 256 merges of n = 32: S 48 -> 42, T 97 -> 78 us; S and
 // T of 1,024 leaves of 32^2: 2.32 -> 1.79 ms.  Of that: one block in flight instead of two 604 us
 // for the n = 512 product; workgroups in launch order, so that each XCD's L2 sees every tile, 578.
-// Each element sums its k range in the same order as there.
+// Each element sums its k range in tree_gemm_kernel's order.
 template <int WR, int WC>
 __global__ void __launch_bounds__(256) tree_gemm_lds_kernel(const TreeGemm* __restrict__ probs,
                                                             const int* __restrict__ start,
@@ -563,15 +563,6 @@ __global__ void __launch_bounds__(1024) tree_gemm_split_kernel(const TreeGemm* _
 // ---------------------------------------------------------------------------------------
 // Gauss-Jordan inversion
 // ---------------------------------------------------------------------------------------
-// Tournament LU of the panel (columns k .. k+nb) with partial pivoting, fused with the step's
-// pivot bookkeeping.  One workgroup of 64 WAVES threads holds up to 32 WAVES panel rows, each row
-// in two adjacent lanes (16 columns each) in registers.  STAGE 0: the rows of chunk blockIdx.x
-// (positions k + ch * rows + i); STAGE 1: the candidates of every chunk (a.cand).  Ties go to
-// the lower position, as idamax takes the first maximum.  FIN = false: the nb rows pivoted on,
-// in order, are the chunk's candidates.  FIN = true (one chunk, or stage 1): they are the pivots
-// of the step, and the same workgroup forms P^-1 of the pivot block from the rows it published
-// (the multiplier of each eliminated entry is kept in place, so the pivot row of column J holds
-// row J of [L11 \ U11]), the LAPACK-order interchanges (ipiv) and the position -> row map (src).
 // Tournament LU of the panel (columns k .. k+nb) with partial pivoting, fused with the step's
 // pivot bookkeeping.  One workgroup of 64 WAVES threads holds up to 64 WAVES RPL panel rows,
 // RPL whole rows (32 columns) per lane in registers, row q NT + tid of the chunk in slot q.

@@ -63,7 +63,7 @@ __host__ __device__ inline int child_src_r(int c, int s) {
 // ---------------------------------------------------------------------------------------
 // Batched two-segment GEMM on v_mfma_f64_16x16x4_f64, row-major operands:
 //   D = alpha0 A0 B0 + alpha1 A1 B1 + beta C        (segment 1 absent when K1 == 0,
-//                                                    C absent when null)
+//                                                    C absent when null; alpha 1 or -1)
 // A0 is M x K0 (lda0), B0 is K0 x N (ldb0), ...  C may alias D (read, then written, by the
 // same lane).  One wave computes a (16 RT) x (16 TN) block; the blocks of all problems of a
 // launch form one flat list (problem p owns waves start[p] .. start[p+1]-1).
@@ -179,10 +179,9 @@ __global__ void inv_update_kernel(const double* Wa, double* Wb, const double* Mm
 struct AsmDesc {
     const double* Tc[4];
     double* X;
-    double* T;
     int n, pad;
 };
-static_assert(sizeof(AsmDesc) == 56, "AsmDesc layout");
+static_assert(sizeof(AsmDesc) == 48, "AsmDesc layout");
 __global__ void tree_assemble_kernel(const AsmDesc* d);
 
 // coarsen_ (HPSAlgorithm.hpp:707-741): dst (4 m/2 square) = blkdiag4(L21) src (4m square) blkdiag4(L12)

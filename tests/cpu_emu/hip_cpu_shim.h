@@ -155,16 +155,7 @@ inline emu_u2 __builtin_amdgcn_permlane32_swap(unsigned old, unsigned src, bool,
     const unsigned from_old = (unsigned)__shfl((double)old, l ^ 32);
     return {{l >= 32 ? from_src : old, l < 32 ? from_old : src}};
 }
-// v_permlane16_swap: rows 1 and 3 (of 16 lanes) of the first operand trade places with rows 0
-// and 2 of the second
-inline emu_u2 __builtin_amdgcn_permlane16_swap(unsigned old, unsigned src, bool, bool) {
-    const int l = (int)(threadIdx.x % 64);
-    const unsigned from_src = (unsigned)__shfl((double)src, l ^ 16);
-    const unsigned from_old = (unsigned)__shfl((double)old, l ^ 16);
-    return {{(l & 16) ? from_src : old, (l & 16) ? src : from_old}};
-}
 // v_mov_b32 with a DPP source (the controls the product uses): quad_perm, row_shl/row_shr 1..15,
-// row_newbcast:0..15 (lane i of the own row),
 // row_bcast:15 (lane 15 of the previous row) and row_bcast:31 (lane 31, rows 2 and 3).  Lanes
 // in rows or banks masked off keep `old`; lanes without a source lane get 0 with bound_ctrl, else `old`.
 inline int __builtin_amdgcn_update_dpp(int old, int src, int ctrl, int row_mask, int bank_mask, bool bound_ctrl) {
@@ -173,7 +164,6 @@ inline int __builtin_amdgcn_update_dpp(int old, int src, int ctrl, int row_mask,
     if (ctrl >= 0 && ctrl <= 0xff) s = (l & ~3) | ((ctrl >> (2 * (l & 3))) & 3);
     else if (ctrl >= 0x101 && ctrl <= 0x10f) { if (i + (ctrl - 0x100) < 16) s = l + (ctrl - 0x100); }
     else if (ctrl >= 0x111 && ctrl <= 0x11f) { if (i - (ctrl - 0x110) >= 0) s = l - (ctrl - 0x110); }
-    else if (ctrl >= 0x150 && ctrl <= 0x15f) s = 16 * r + (ctrl - 0x150);
     else if (ctrl == 0x142) { if (r >= 1) s = 16 * r - 1; }
     else if (ctrl == 0x143) { if (r >= 2) s = 31; }
     else { fprintf(stderr, "emulator: DPP control 0x%x not modelled\n", ctrl); abort(); }
@@ -182,20 +172,6 @@ inline int __builtin_amdgcn_update_dpp(int old, int src, int ctrl, int row_mask,
     if (s < 0) return bound_ctrl ? 0 : old;
     return v;
 }
-// its 64-bit form (v_mov_b64_dpp): row_newbcast only, on every lane
-inline long long __builtin_amdgcn_update_dpp(long long, long long src, int ctrl, int row_mask, int bank_mask, bool) {
-    if (ctrl < 0x150 || ctrl > 0x15f || row_mask != 0xf || bank_mask != 0xf) {
-        fprintf(stderr, "emulator: 64-bit DPP control 0x%x not modelled\n", ctrl);
-        abort();
-    }
-    double x;
-    std::memcpy(&x, &src, 8);
-    x = __shfl(x, (int)(threadIdx.x % 64) / 16 * 16 + (ctrl - 0x150));
-    std::memcpy(&src, &x, 8);
-    return src;
-}
-inline long long __double_as_longlong(double x) { long long u; std::memcpy(&u, &x, 8); return u; }
-inline double __longlong_as_double(long long u) { double x; std::memcpy(&x, &u, 8); return x; }
 inline double __builtin_amdgcn_rcp(double x) { return 1.0 / x; }
 // a scheduling barrier on the GPU (lanes of a wave run in lockstep); here the lanes meet
 #define __builtin_amdgcn_wave_barrier() emu_wave_sync()
