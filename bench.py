@@ -38,11 +38,11 @@ BOUNDS = (-10.0, 10.0, -10.0, 10.0)
 METRIC = "solves/s + p50/p99 latency at 1e-8 rel err vs FP64; buildStage seconds"
 # HBM bytes per launch measured by two rocprofv3 counter passes (FETCH_SIZE x 2.0 +
 # WRITE_SIZE x 1.0, factors from the copy kernel); profiles/patch_fd_kernel_adaptive_poisson_leafset.md and
-# profiles/bt_solve_sym_kernel_variable_beta_leafset.md have the commands and the raw values.
+# profiles/bt_solve_mfma_kernel_variable_beta_leafset.md have the commands and the raw values.
 TRAFFIC_PER_LAUNCH = 572.9e6          # leaf solves of this workload, 16 right-hand sides
 TRAFFIC_MAP_D2N = 319.0e6             # particular Neumann data, same leaf set and k
-TRAFFIC_VAR_BETA = 1329.8e6           # variable-beta leaf solves, packed symmetric blocks
-TRAFFIC_GEMM_PER_LAUNCH = 135.36e6    # tree_gemm_kernel in the sweep at 64 columns, per launch: profiles/tree_gemm_kernel_adaptive_poisson_sweep.md
+TRAFFIC_VAR_BETA = 1305.2e6           # variable-beta leaf solves, packed symmetric blocks
+TRAFFIC_GEMM_PER_LAUNCH = 133.71e6    # tree_gemm_kernel in the sweep at 64 columns, per launch: profiles/tree_gemm_kernel_adaptive_poisson_sweep.md
 
 
 def log(msg):
