@@ -1511,8 +1511,8 @@ void do_solve_once(ef_mesh_s* M, const double* f_dev, const double* r_dev, const
         const double* hroot = (root.leaf || M->homogeneous_rhs) ? nullptr : V + root.h_off;
         int info[2] = {0, 0};  // zero pivot, stop of the natural order
         EF_HIP(hipMemsetAsync(M->rootinfo.p, 0, 2 * sizeof(int), s));
-        EF_LAUNCH("tree_root_robin_kernel", tree_root_robin_kernel, dim3(blocks_for((long long)m * m + (long long)m * k)),
-                  dim3(256), s, Troot, a_dev, b_dev, r_dev, hroot, M->rootA.p, M->rootrhs.p, m, k, P.vec_rows);
+        EF_LAUNCH("tree_root_robin_kernel", tree_root_robin_kernel, dim3(m), dim3(256), s, Troot, a_dev, b_dev, r_dev, hroot,
+                  M->rootA.p, M->rootrhs.p, m, k, P.vec_rows);
         run_inverse(M->rootA.p, M->rootAi.p, m, 1, M->rootgj.p, M->rootinfo.p + 1, s);
         efk::copy_d2h(info, M->rootinfo.p, 2 * sizeof(int), s);
         if (info[1]) {  // on with row exchanges, from the buffer the natural order left the matrix in to the other

@@ -46,6 +46,37 @@ def root_case(ctx, N, level, lam, kind, ks=(1, 5, 1)):
     return O, a, b
 
 
+def rebuild_case(ctx, N, level, ks):
+    """One mesh built again: the root's system is formed from the new T, and its product's plan, kept where no address
+    moved, reads the new inverse."""
+    import ellipticforest_amd as ef
+    leaves, bounds = omesh.uniform(level), (-1, 1, -1, 1)
+    D = ef.DeviceMesh(ctx, leaves, N, bounds)
+    a, b = root_rows(4 * D.M, "plus")
+    rng = np.random.default_rng(N)
+    for lam in (-1.0, -30.0, -1.0):
+        O = oracle.Forest(leaves, N, bounds, solver=oracle.FISHPACK, lambda0=lam)
+        O.build()
+        D.build(lambda0=lam)
+        for k in ks:
+            f, r = rng.standard_normal((k, D.nleaves, N * N)), rng.standard_normal((k, 4 * D.M))
+            D.upwards(f)
+            u = D.solve(r, a, b)
+            for c in range(k):
+                O.upwards(f[c])
+                assert gp.rel(u[c], O.solve(r[c], a, b)) < gp.TOL_U, (lam, k, c)
+
+
+@pytest.mark.gpu
+def test_root_after_rebuild(ctx):
+    gp.say("Robin roots of one mesh built again, order 160")
+    rebuild_case(ctx, 20, 1, (1, 3))
+
+
+def test_emu_root_after_rebuild(emu_ctx):
+    rebuild_case(emu_ctx, 4, 1, (1,))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("N,level,kind", [(8, 1, "far"), (20, 1, "far"), (20, 1, "rows"), (20, 1, "plus")])
 def test_root_rows(ctx, N, level, kind):
